@@ -237,6 +237,7 @@ int launch_site_energies(graspa_box* b, const SiteBatch& sb, int self_comp, int 
 int launch_ewald_delta(graspa_box* b, const SiteBatch& sb, int n_old, double* d_out /* blocks*2 */, int* n_blocks);
 int launch_ewald_build(graspa_box* b, double* d_out_energy /* blocks*3 */, int* n_blocks);
 int launch_total_pairs(graspa_box* b, double* d_out /* blocks*4 */, int* n_blocks);
+int launch_fourier_total(graspa_box* b, double* d_out /* blocks*3 */, int* n_blocks);
 
 // writes atoms [first_atom, first_atom + n_atoms) of a component from the host
 // mirror into the device guest store (engine_api.hip)

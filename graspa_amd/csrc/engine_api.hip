@@ -935,11 +935,15 @@ int graspa_total_energy(graspa_box* b, graspa_energy* e)
   hipSetDevice(b->device);
   GuestView gv;
   guest_view(b, &gv);
-  const int nb_max = (std::max(gv.total, 1) + kBlock - 1) / kBlock;
-  if (int rc = ensure_part(b, 4 * (size_t)nb_max + 8)) return rc;
-  int nb = 0;
+  // one partial per guest atom (pair sums) and per kBlock active k-vectors
+  // (Fourier sums), read back in one copy
+  const size_t n_pair = 4 * (size_t)gv.total, n_four = 3 * (size_t)((b->n_active + kBlock - 1) / kBlock);
+  if (int rc = ensure_part(b, n_pair + n_four + 8)) return rc;
+  int nb = 0, nk = 0;
   if (int rc = launch_total_pairs(b, b->d_part, &nb)) return rc;
-  if (hip_check(hipMemcpyAsync(b->h_part, b->d_part, 4 * nb * sizeof(double), hipMemcpyDeviceToHost, b->stream),
+  if (int rc = launch_fourier_total(b, b->d_part + n_pair, &nk)) return rc;
+  if (hip_check(hipMemcpyAsync(b->h_part, b->d_part, (n_pair + n_four) * sizeof(double), hipMemcpyDeviceToHost,
+                               b->stream),
                 "total copy"))
     return GRASPA_ERR_HIP;
   if (hip_check(hipStreamSynchronize(b->stream), "total sync")) return GRASPA_ERR_HIP;
@@ -950,17 +954,10 @@ int graspa_total_energy(graspa_box* b, graspa_energy* e)
     e->gg_vdw += b->h_part[4 * i + 2];
     e->gg_real += b->h_part[4 * i + 3];
   }
-  // Fourier part from the running structure factors
-  std::vector<double2> sf(b->nvec), sa(b->nvec);
-  if (hip_check(hipMemcpy(sf.data(), b->d_sk_fw, b->nvec * sizeof(double2), hipMemcpyDeviceToHost), "sk copy") ||
-      hip_check(hipMemcpy(sa.data(), b->d_sk_ads, b->nvec * sizeof(double2), hipMemcpyDeviceToHost), "sk copy"))
-    return GRASPA_ERR_HIP;
-  for (int k = 0; k < b->nvec; ++k) {
-    const double t = b->ktemp[k];
-    if (t < 0.0) continue;
-    e->gg_ewald += t * (sa[k].x * sa[k].x + sa[k].y * sa[k].y);
-    e->hh_ewald += t * (sf[k].x * sf[k].x + sf[k].y * sf[k].y);
-    e->hg_ewald += t * (sf[k].x * sa[k].x + sf[k].y * sa[k].y) * 2.0;
+  for (int i = 0; i < nk; ++i) {
+    e->gg_ewald += b->h_part[n_pair + 3 * i];
+    e->hh_ewald += b->h_part[n_pair + 3 * i + 1];
+    e->hg_ewald += b->h_part[n_pair + 3 * i + 2];
   }
   return GRASPA_OK;
 }
