@@ -303,6 +303,9 @@ void build_coulomb_table(double alpha, double cut2, std::vector<double>& tab);
 // widom_kernel.hip
 // Bytes of the no-allocation form's fixed scratch block (one per device).
 constexpr size_t kWidomScratchBytes = (size_t)32 << 20;
+// ... and room behind it for the slots that the screening grid rounds up to:
+// at most one insertion per workgroup, i.e. 1,024 of 56 K + 56 O (M - 1) + 64 bytes (K <= 32, O (M - 1) <= 64)
+constexpr size_t kWidomScratchSlack = (size_t)8 << 20;
 // How a Widom batch is launched.  no_alloc: the pipeline's scratch comes
 // from that block, and no buffer or voxel map is allocated (maps built by
 // earlier calls are used).  first_dev: the batch's first insertion index is

@@ -1407,18 +1407,22 @@ struct WidomBufs {
 };
 
 // Screening grid of a batch: up to kMaxScreenGroups workgroups, each owning
-// a contiguous range of `chunk` insertions (four wave steps of kFbWaves x 64 /
-// K insertions each); the work lists and the live list have a sub-list of
-// chunk insertions per workgroup.  The first-bead, chain and finish kernels
-// hold one workgroup per CU, so the group count is rounded down to a
-// multiple of the CU count: a few groups beyond it would take a second round
-// of the whole kernel.
+// a contiguous range of `chunk` insertions; the work lists and the live list
+// have a sub-list of chunk insertions per workgroup.  The first-bead, chain
+// and finish kernels hold one workgroup per CU, so a batch gets one for each
+// CU down to eight insertions a workgroup (at 384 insertions a workgroup,
+// 1,000 insertions ran on 3 CUs and 20,000 on 53: the three kernels took 31 /
+// 113 / 110 us of a batch of 1,000 and 42 / 145 / 365 us of a batch of 20,000
+// in a loaded box, now 11 / 18 / 18 and 18 / 38 / 274 us); a batch of more
+// than 384 a CU gets a multiple of the CU count: a few groups beyond it would
+// take a second round of the whole kernel.
 static void widom_grid(const graspa_box* b, int K, int n_insert, int* groups, int* chunk)
 {
   const long long per_group = 4LL * kFbWaves * (64 / K);
-  long long raw = std::max<long long>(1, ((long long)n_insert + per_group - 1) / per_group);
   const long long ncu = std::max(1, b->n_cu);
+  long long raw = std::max<long long>(1, ((long long)n_insert + per_group - 1) / per_group);
   if (raw > ncu) raw = raw / ncu * ncu;
+  raw = std::max(raw, std::min<long long>(ncu, ((long long)n_insert + 7) / 8));
   const long long cap = kMaxScreenGroups >= ncu ? kMaxScreenGroups / ncu * ncu : kMaxScreenGroups;
   *groups = (int)std::min<long long>(raw, cap);
   *chunk = (n_insert + *groups - 1) / *groups;
@@ -1482,7 +1486,7 @@ static size_t carve_bufs(char* base, int n_insert, int K, int OC, int n_slots, W
 // once per device with hipGetSymbolAddress (host code never uses the
 // symbol's name as an address).  Shared by every call on the device.
 constexpr int kMaxDevices = 64;
-static __device__ __align__(256) char widom_scratch[kWidomScratchBytes];
+static __device__ __align__(256) char widom_scratch[kWidomScratchBytes + kWidomScratchSlack];
 static std::mutex scratch_mu;
 static char* scratch_ptr[kMaxDevices];   // per device, null until looked up
 
@@ -1539,7 +1543,14 @@ int launch_widom(graspa_box* b, int comp, int K, int O, double beta, int bias, d
     W.rec_f = b->d_wrec_f;
     W.part = b->d_wpart;
   } else if (how.no_alloc) {
-    const size_t need = carve_bufs(nullptr, n_insert, K, O * chain, groups * chunk, nullptr);
+    // (the limit counts the slots of whole wave steps, 4 kFbWaves (64 / K)
+    // insertions a workgroup, whatever the grid; the block has room for the
+    // few slots more that a grid of one workgroup per CU rounds up to)
+    const long long step = 4LL * kFbWaves * (64 / K), ncu = std::max(1, b->n_cu);
+    long long g = ((long long)n_insert + step - 1) / step;
+    if (g > ncu) g = g / ncu * ncu;
+    g = std::min<long long>(g, kMaxScreenGroups >= ncu ? kMaxScreenGroups / ncu * ncu : kMaxScreenGroups);
+    const size_t need = carve_bufs(nullptr, n_insert, K, O * chain, (int)(g * (((long long)n_insert + g - 1) / g)), nullptr);
     if (need > (size_t)kWidomScratchBytes)
       return fail(GRASPA_ERR_ARG, "widom (no allocation): the batch needs " + std::to_string(need) +
                                       " bytes of scratch, above the fixed " + std::to_string(kWidomScratchBytes) +
