@@ -139,6 +139,14 @@ struct graspa_box {
   double2* d_sk_stage = nullptr;
   int4* d_kact = nullptr;       // active k-vectors: kx, ky, kz, index
   double* d_ktemp_act = nullptr;  // ktemp of the active k-vectors
+  // the active k-vectors as rows (kx, ky) of k_z, -k_z pairs, 64 rows to a
+  // chunk (layout: WidomArgs), and the Widom finish kernel's coefficients
+  int n_kchunk = 0, n_kpack = 0;
+  int2* d_kchunk = nullptr;
+  int* d_krow = nullptr;
+  double2* d_kt = nullptr;
+  int2* d_kidx = nullptr;
+  double4* d_ku = nullptr;
   std::vector<double> ktemp;
   bool sk_staged = false;
 
@@ -263,6 +271,8 @@ __host__ __device__ inline double overlap_r2(double a4e, double s2, double shift
   return thr < cut2 ? thr : cut2;
 }
 
+// rows of the active k-vectors (engine_api.hip)
+int build_k_rows(graspa_box* b);
 // screen cell grid of the framework (engine_api.hip)
 int build_screen_cells(graspa_box* b);
 

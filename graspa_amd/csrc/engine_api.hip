@@ -294,6 +294,62 @@ int graspa::build_screen_cells(graspa_box* b)
   return GRASPA_OK;
 }
 
+// The active k-vectors grouped by row (kx, ky): rows in descending order of
+// their largest |kz|, so that the 64 rows of a chunk have about the same.
+int graspa::build_k_rows(graspa_box* b)
+{
+  const int kxm = b->bc.kmax[0], kym = b->bc.kmax[1], kzm = b->bc.kmax[2];
+  auto index = [&](int kx, int ky, int kz) { return (kx * (2 * kym + 1) + ky + kym) * (2 * kzm + 1) + kz + kzm; };
+  struct Row {
+    int kx, ky, top;
+  };
+  std::vector<Row> rows;
+  for (int kx = 0; kx <= kxm; ++kx)
+    for (int ky = -kym; ky <= kym; ++ky) {
+      int top = -1;
+      for (int kz = 0; kz <= kzm; ++kz)
+        if (b->ktemp[index(kx, ky, kz)] >= 0.0 || b->ktemp[index(kx, ky, -kz)] >= 0.0) top = kz;
+      if (top >= 0) rows.push_back(Row{kx, ky, top});
+    }
+  std::stable_sort(rows.begin(), rows.end(), [](const Row& x, const Row& y) { return x.top > y.top; });
+  const int nch = ((int)rows.size() + 63) / 64;
+  std::vector<int2> chunk(std::max(nch, 1), make_int2(0, 0));
+  std::vector<int> row(64 * (size_t)std::max(nch, 1), 64 << 8);
+  int n = 0;
+  for (int c = 0; c < nch; ++c) {
+    chunk[c] = make_int2(n, rows[64 * c].top);
+    n += 64 * (rows[64 * c].top + 1);
+  }
+  std::vector<double2> kt((size_t)std::max(n, 1), make_double2(0.0, 0.0));
+  std::vector<int2> idx((size_t)std::max(n, 1), make_int2(-1, -1));
+  for (size_t r = 0; r < rows.size(); ++r) {
+    row[r] = rows[r].kx | ((rows[r].ky + 64) << 8);
+    for (int kz = 0; kz <= rows[r].top; ++kz) {
+      const size_t e = (size_t)chunk[r / 64].x + 64 * (size_t)kz + r % 64;
+      const int kp = index(rows[r].kx, rows[r].ky, kz), km = index(rows[r].kx, rows[r].ky, -kz);
+      if (b->ktemp[kp] >= 0.0) {
+        idx[e].x = kp;
+        kt[e].x = b->ktemp[kp];
+      }
+      if (kz > 0 && b->ktemp[km] >= 0.0) {
+        idx[e].y = km;
+        kt[e].y = b->ktemp[km];
+      }
+    }
+  }
+  b->n_kchunk = nch;
+  b->n_kpack = n;
+  int rc = hip_check(box_malloc(b, &b->d_kchunk, chunk.size() * sizeof(int2)), "hipMalloc k rows");
+  rc = rc ? rc : hip_check(box_malloc(b, &b->d_krow, row.size() * sizeof(int)), "hipMalloc k rows");
+  rc = rc ? rc : hip_check(box_malloc(b, &b->d_kt, kt.size() * sizeof(double2)), "hipMalloc k rows");
+  rc = rc ? rc : hip_check(box_malloc(b, &b->d_kidx, idx.size() * sizeof(int2)), "hipMalloc k rows");
+  rc = rc ? rc : hip_check(box_malloc(b, &b->d_ku, kt.size() * sizeof(double4)), "hipMalloc k rows");
+  rc = rc ? rc : hip_check(hipMemcpy(b->d_kchunk, chunk.data(), chunk.size() * sizeof(int2), hipMemcpyHostToDevice), "k rows upload");
+  rc = rc ? rc : hip_check(hipMemcpy(b->d_krow, row.data(), row.size() * sizeof(int), hipMemcpyHostToDevice), "k rows upload");
+  rc = rc ? rc : hip_check(hipMemcpy(b->d_kt, kt.data(), kt.size() * sizeof(double2), hipMemcpyHostToDevice), "k rows upload");
+  return rc ? rc : hip_check(hipMemcpy(b->d_kidx, idx.data(), idx.size() * sizeof(int2), hipMemcpyHostToDevice), "k rows upload");
+}
+
 #define GRASPA_CHECK_BOX(b) \
   if (!(b)) return fail(GRASPA_ERR_ARG, "null box");
 
@@ -463,6 +519,7 @@ int graspa_box_create(const graspa_box_params* p, graspa_box** out)
                           "k upload");
     }
   }
+  if (!rc) rc = build_k_rows(b);
   {
     // real-space Coulomb table of the fast form
     std::vector<double> ct(kCoulTabStride, 0.0);
@@ -506,6 +563,7 @@ void graspa_box_destroy(graspa_box* b)
   box_free(b, b->d_fws); box_free(b, b->d_fws_type); box_free(b, b->d_ctab);
   box_free(b, b->d_g); box_free(b, b->d_g_type); box_free(b, b->d_g_molid); box_free(b, b->d_g_comp); box_free(b, b->d_g_fix);
   box_free(b, b->d_ktemp); box_free(b, b->d_sk_fw); box_free(b, b->d_sk_ads); box_free(b, b->d_sk_stage);
+  box_free(b, b->d_kchunk); box_free(b, b->d_krow); box_free(b, b->d_kt); box_free(b, b->d_kidx); box_free(b, b->d_ku);
   box_free(b, b->d_kact); box_free(b, b->d_ktemp_act); box_free(b, b->d_coul);
   free_dead_maps(b);
   for (Component& c : b->comps) box_free(b, c.d_chain);

@@ -18,11 +18,12 @@ __device__ inline double2 cmul2(double2 a, double2 b)
 // three uniforms (Shoemake's quaternion).
 __device__ inline void quat_rotate(double v[3], double u, double vv, double w)
 {
-  const double pi = 3.14159265358979323846;
-  const double q0 = sqrt(1 - u) * sin(2 * pi * vv);
-  const double q1 = sqrt(1 - u) * cos(2 * pi * vv);
-  const double q2 = sqrt(u) * sin(2 * pi * w);
-  const double q3 = sqrt(u) * cos(2 * pi * w);
+  // (sin and cos of 2 pi x by sincospi: its reduction is exact and short)
+  double s1, c1, s2, c2;
+  sincospi(2.0 * vv, &s1, &c1);
+  sincospi(2.0 * w, &s2, &c2);
+  const double a = sqrt(1 - u), b = sqrt(u);
+  const double q0 = a * s1, q1 = a * c1, q2 = b * s2, q3 = b * c2;
   const double a01 = q0 * q1, a02 = q0 * q2, a03 = q0 * q3;
   const double a11 = q1 * q1, a12 = q1 * q2, a13 = q1 * q3;
   const double a22 = q2 * q2, a23 = q2 * q3, a33 = q3 * q3;
@@ -61,11 +62,10 @@ __device__ inline void axis_table(const BoxConst& bc, double px, double py, doub
   if (axis == 0) s = a[0] * px + a[3] * py + a[6] * pz;
   else if (axis == 1) s = a[1] * px + a[4] * py + a[7] * pz;
   else s = a[2] * px + a[5] * py + a[8] * pz;
-  s *= 2 * 3.14159265358979323846;
   const int km = bc.kmax[axis];
   out[0] = make_double2(1.0, 0.0);
   double sn, cs;
-  sincos(s, &sn, &cs);
+  sincospi(2.0 * s, &sn, &cs);
   const double2 e1 = make_double2(cs, sn);
   if (km >= 1) out[1] = e1;
   // the running power stays in registers (out may be LDS: no store-to-load

@@ -126,6 +126,14 @@ struct WidomArgs {
   const double2* sk_ads;
   const double2* sk_fw;
   int kstride;              // max kmax + 1
+  // the active k-vectors as rows (kx, ky), 64 to a chunk, entry first + 64 kz
+  // + lane of a chunk holding those of k_z and -k_z
+  int n_kchunk, n_kpack;
+  const int2* kchunk;       // first entry, largest kz
+  const int* krow;          // kx | (ky + 64) << 8
+  const double2* kt;        // ktemp of k_z, -k_z (0: not active)
+  const int2* kidx;         // their indices in the S(k) arrays (-1: not active)
+  double4* ku;              // 2 ktemp (S_ads + S_fw) of both, by the chain kernel
   const double* coul;       // real-space Coulomb table (fast form)
   int coul_n;               // doubles
   // pipeline buffers
@@ -855,6 +863,22 @@ template <bool CUBIC>
 __global__ __launch_bounds__(kInsWaves * 64) void widom_chain_kernel(const WidomArgs A)
 {
   extern __shared__ __align__(16) char dyn[];
+  // the finish kernel's Fourier coefficients of the current structure factors
+  if (A.charged)
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < A.n_kpack; i += gridDim.x * blockDim.x) {
+      const int2 k = A.kidx[i];
+      const double2 t = A.kt[i];
+      double4 u = make_double4(0.0, 0.0, 0.0, 0.0);
+      if (k.x >= 0) {
+        u.x = 2.0 * t.x * (A.sk_ads[k.x].x + A.sk_fw[k.x].x);
+        u.y = 2.0 * t.x * (A.sk_ads[k.x].y + A.sk_fw[k.x].y);
+      }
+      if (k.y >= 0) {
+        u.z = 2.0 * t.y * (A.sk_ads[k.y].x + A.sk_fw[k.y].x);
+        u.w = 2.0 * t.y * (A.sk_ads[k.y].y + A.sk_fw[k.y].y);
+      }
+      A.ku[i] = u;
+    }
   __shared__ unsigned wg_cnt, wg_pl;
   __shared__ unsigned long long wg_st;
   const int T = A.bc.ntypes;
@@ -1033,8 +1057,240 @@ __global__ __launch_bounds__(kInsWaves * 64) void widom_chain_kernel(const Widom
 // and the record: W = W_fb W_ch exp(-beta (dE_ewald + dE_tail)), for the
 // insertions whose first bead was placed (the others have their records from
 // the first-bead or the chain kernel).  gridDim.x / groups workgroups share
-// the placed list of screening workgroup g, one wave per insertion.
-__global__ __launch_bounds__(kFinWaves * 64) void widom_finish_kernel(const WidomArgs A)
+// the placed list of screening workgroup g.
+//
+// A wave takes four insertions at a time, one per 16-lane row in the
+// selection.  The Fourier sum then runs over rows (kx, ky) of k-vectors, one
+// per lane, for the four together: q e^{i(kx x + ky y)} of a row stays in
+// registers, and the products of its real and imaginary part with those of
+// e^{i kz z} (read by all lanes at one LDS address) give both k_z and -k_z:
+// 26 instructions for two k-vectors of a three-site molecule, against 2 x 55
+// with one k-vector per lane.  t |S + c|^2 - t |S|^2 + 2 t S_fw . c is taken
+// as U . c + t |c|^2 with U = 2 t (S + S_fw) from the chain kernel, in the
+// lanes' order (48 bytes per k-vector pair, read once for four insertions):
+// with 56 gathered bytes per k-vector and insertion the kernel was bound by
+// L2, 106 KB per insertion of a 40 x 40 x 27 A box (366 us of 20,000
+// insertions there, 406 us of 100,000 in a 24 A box, at a workgroup per CU 274
+// and 400; now 99 and 163).
+// M: sites per molecule (their row products are in registers).
+template <int M>
+__global__ __launch_bounds__(kFinWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void widom_finish_kernel(const WidomArgs A)
+{
+  extern __shared__ __align__(16) char dyn[];
+  const BoxConst& bc = A.bc;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, row = lane >> 4, rl = lane & 15;
+  const int K = A.K, O = A.O, KS = A.kstride;
+  constexpr int chain = M - 1;
+  constexpr int kIns = 4;
+  // per wave: axis tables [insertion][site][axis][KS], positions [insertion][site][3]
+  const size_t wave_bytes = (size_t)kIns * M * 3 * (KS * sizeof(double2) + sizeof(double));
+  double2* eik = reinterpret_cast<double2*>(dyn + (size_t)wv * wave_bytes);
+  double* mol = reinterpret_cast<double*>(eik + (size_t)kIns * M * 3 * KS);
+  const int per = gridDim.x / A.groups, g = blockIdx.x / per, part = blockIdx.x - g * per;
+  const unsigned n_pl = A.placed_counts[g];
+  const int* placed = A.placed + (size_t)g * A.chunk;
+  // one, two or four insertions at a time, as many as keep every wave busy
+  // (a wave's step with four takes three times as long as with one)
+  const unsigned waves = (unsigned)(per * kFinWaves);
+  const unsigned take = n_pl <= waves ? 1u : (n_pl <= 2u * waves ? 2u : 4u);
+  for (unsigned k = (unsigned)(part * kFinWaves + wv) * take; k < n_pl; k += waves * take) {
+    const bool has = (unsigned)row < take && k + row < n_pl;
+    const int ins = placed[has ? k + row : k];
+    const uint64_t idx = (uint64_t)(first_of(A) + ins);
+    const InsState S = A.state[ins];
+    bool ok = has && S.ok != 0;
+    double Wtot = S.wfb, e_v = S.ev, e_r = S.er;
+    int orient = 0;
+    if constexpr (chain > 0) {
+      const uint32_t dead2 = A.mask2[ins];
+      const double u = draw(A, idx, 3 * K + 3 * O + 1);
+      int so = -1;
+      double Wch = 0.0, sv = 0.0, sr = 0.0;
+      if (O <= 16) {
+        const bool alive = ok && rl < O && !((dead2 >> rl) & 1u);
+        double cv = 0.0, cr = 0.0;
+        // (dropped trials' energies are read too, so that the loads need not
+        // wait for the masks)
+        double2 e[chain];
+#pragma unroll
+        for (int a = 0; a < chain; ++a) e[a] = A.e2[((size_t)ins * O + (rl < O ? rl : 0)) * chain + a];
+#pragma unroll
+        for (int a = 0; a < chain; ++a) {
+          cv += alive ? e[a].x : 0.0;
+          cr += alive ? e[a].y : 0.0;
+        }
+        row_select(cv, cr, alive, O, u, A.beta, A.bias, so, Wch);
+        const int sl = row * 16 + (so >= 0 ? so : 0);
+        sv = __shfl(cv, sl, 64);
+        sr = __shfl(cr, sl, 64);
+      } else {
+        for (int q = 0; q < kIns; ++q) {
+          const int ins_q = __builtin_amdgcn_readlane(ins, 16 * q);
+          const uint32_t dead_q = (uint32_t)__builtin_amdgcn_readlane((int)dead2, 16 * q);
+          double cv = 0.0, cr = 0.0;
+          if (lane < O && !((dead_q >> lane) & 1u)) {
+            for (int a = 0; a < chain; ++a) {
+              const double2 e = A.e2[((size_t)ins_q * O + lane) * chain + a];
+              cv += e.x;
+              cr += e.y;
+            }
+          }
+          int so_q;
+          double W_q;
+          wave_select(cv, cr, dead_q, O, readlane_d(u, 16 * q), A.beta, A.bias, so_q, W_q);
+          const double sv_q = readlane_d(cv, so_q >= 0 ? so_q : 0), sr_q = readlane_d(cr, so_q >= 0 ? so_q : 0);
+          if (row == q) {
+            so = so_q;
+            Wch = W_q;
+            sv = sv_q;
+            sr = sr_q;
+          }
+        }
+      }
+      if (so < 0 || !(S.wfb * Wch > 1e-150)) {
+        ok = false;
+      } else {
+        Wtot = S.wfb * Wch;
+        orient = so;
+        e_v += sv;
+        e_r += sr;
+      }
+    }
+    double ew = 0.0;
+    if (A.charged && __any(ok)) {
+      if (rl < M) {
+        double p[3] = {S.fb[0], S.fb[1], S.fb[2]};
+        if constexpr (chain > 0)
+          if (rl > 0) {
+            double u[3];
+            draw3(A, idx, 3 * K + 1 + 3 * orient, u);
+            double vec[3] = {A.tvec[rl - 1][0], A.tvec[rl - 1][1], A.tvec[rl - 1][2]};
+            quat_rotate(vec, u[0], u[1], u[2]);
+            p[0] = S.fb[0] + vec[0];
+            p[1] = S.fb[1] + vec[1];
+            p[2] = S.fb[2] + vec[2];
+          }
+        double* q = mol + (row * M + rl) * 3;
+        q[0] = p[0]; q[1] = p[1]; q[2] = p[2];
+      }
+      wave_sync();
+      for (int t = lane; t < (int)take * M * 3; t += 64) {
+        const int sm = t / 3, axis = t - 3 * sm;
+        axis_table(bc, mol[3 * sm], mol[3 * sm + 1], mol[3 * sm + 2], axis, eik + (size_t)t * KS);
+      }
+      wave_sync();
+      double es[kIns] = {0.0, 0.0, 0.0, 0.0};
+      auto fourier = [&](auto n_c) {
+      constexpr int N = decltype(n_c)::value;
+      for (int ch = 0; ch < A.n_kchunk; ++ch) {
+        const int2 kc = A.kchunk[ch];            // first entry, largest kz
+        const int kr = A.krow[64 * ch + lane];
+        const int kx = kr & 0xff, ky = (kr >> 8) - 64;
+        double2 exy[N][M];
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+#pragma unroll
+          for (int s = 0; s < M; ++s) {
+            const double2* e = eik + (size_t)(i * M + s) * 3 * KS;
+            double2 ey = e[KS + abs(ky)];
+            if (ky < 0) ey.y = -ey.y;
+            const double2 p = cmul2(e[kx], ey);
+            exy[i][s] = make_double2(A.site_q[s] * p.x, A.site_q[s] * p.y);
+          }
+        const double4* U = A.ku + (size_t)kc.x + lane;
+        const double2* tt = A.kt + (size_t)kc.x + lane;
+        {
+          // kz = 0
+          const double4 u = U[0];
+          const double t = tt[0].x;
+#pragma unroll
+          for (int i = 0; i < N; ++i) {
+            double2 c = exy[i][0];
+#pragma unroll
+            for (int s = 1; s < M; ++s) {
+              c.x += exy[i][s].x;
+              c.y += exy[i][s].y;
+            }
+            es[i] = fma(t, fma(c.y, c.y, c.x * c.x), fma(u.y, c.y, fma(u.x, c.x, es[i])));
+          }
+        }
+        auto pair = [&](const int kz, const double4 u, const double2 t) {
+#pragma unroll
+          for (int i = 0; i < N; ++i) {
+            double ac = 0.0, bd = 0.0, ad = 0.0, bc2 = 0.0;
+#pragma unroll
+            for (int s = 0; s < M; ++s) {
+              const double2 ez = eik[((size_t)(i * M + s) * 3 + 2) * KS + kz];
+              ac = fma(exy[i][s].x, ez.x, ac);
+              bd = fma(exy[i][s].y, ez.y, bd);
+              ad = fma(exy[i][s].x, ez.y, ad);
+              bc2 = fma(exy[i][s].y, ez.x, bc2);
+            }
+            const double px = ac - bd, py = ad + bc2, mx = ac + bd, my = bc2 - ad;   // k_z and -k_z
+            double e = fma(u.y, py, fma(u.x, px, es[i]));
+            e = fma(t.x, fma(py, py, px * px), e);
+            e = fma(u.w, my, fma(u.z, mx, e));
+            es[i] = fma(t.y, fma(my, my, mx * mx), e);
+          }
+        };
+        // (with one or two insertions the loads of four steps are issued
+        // together; with four the arithmetic covers them)
+        constexpr int B = N == 4 ? 1 : 4;
+        for (int kz = 1; kz <= kc.y; kz += B) {
+          double4 u[B];
+          double2 t[B];
+#pragma unroll
+          for (int q = 0; q < B; ++q) {
+            const int z = min(kz + q, kc.y);
+            u[q] = U[64 * z];
+            t[q] = tt[64 * z];
+          }
+#pragma unroll
+          for (int q = 0; q < B; ++q)
+            if (kz + q <= kc.y) pair(kz + q, u[q], t[q]);
+        }
+      }
+      };
+      if (take == 1u) fourier(std::integral_constant<int, 1>{});
+      else if (take == 2u) fourier(std::integral_constant<int, 2>{});
+      else fourier(std::integral_constant<int, 4>{});
+#pragma unroll
+      for (int i = 0; i < kIns; ++i) {
+        const double e = wave_sum(es[i]);
+        if (row == i) ew = e - A.excl;
+      }
+      wave_sync();
+    }
+    if (rl == 0 && has) {
+      double Wf = 0.0, etot = 0.0;
+      if (ok) {
+        Wf = Wtot * exp(-A.beta * ew) * exp(-A.beta * A.tail_de);
+        etot = e_v + e_r + ew + A.tail_de;
+      }
+      A.rec_w[ins] = Wf;
+      A.rec_e[ins] = etot;
+      A.rec_f[ins] = (S.ok ? 1 : 0) | (ok ? 2 : 0);
+      if (A.res) {
+        graspa_widom_result r;
+        r.rosen = Wf;
+        r.energy = etot;
+        r.vdw = ok ? e_v : 0.0;
+        r.real = ok ? e_r : 0.0;
+        r.ewald = ok ? ew : 0.0;
+        r.first_bead = ok ? S.sel : -1;
+        r.orientation = ok ? orient : -1;
+        r.ok = ok ? 1 : 0;
+        r._pad = 0;
+        A.res[ins] = r;
+      }
+    }
+  }
+}
+
+// The same for molecules of more than four sites, or axis tables of four
+// insertions that do not fit the LDS: one wave per insertion, one k-vector
+// per lane.
+__global__ __launch_bounds__(kFinWaves * 64) void widom_finish_any_kernel(const WidomArgs A)
 {
   extern __shared__ __align__(16) char dyn[];
   const BoxConst& bc = A.bc;
@@ -1612,6 +1868,9 @@ int launch_widom(graspa_box* b, int comp, int K, int O, double beta, int bias, d
   A.ktemp_act = b->d_ktemp_act;
   A.sk_ads = b->d_sk_ads; A.sk_fw = b->d_sk_fw;
   A.kstride = 1 + std::max(b->bc.kmax[0], std::max(b->bc.kmax[1], b->bc.kmax[2]));
+  A.n_kchunk = b->n_kchunk;
+  A.n_kpack = b->n_kpack;
+  A.kchunk = b->d_kchunk; A.krow = b->d_krow; A.kt = b->d_kt; A.kidx = b->d_kidx; A.ku = b->d_ku;
   A.coul = b->d_coul;
   A.coul_n = b->coul_n;
   A.mask1 = W.mask1;
@@ -1690,14 +1949,20 @@ int launch_widom(graspa_box* b, int comp, int K, int O, double beta, int bias, d
     rc = eval(A.list2, A.counts2, O * chain, A.e2, A.mask2, 1);
     if (rc) return rc;
   }
-  const size_t fin_lds = (size_t)kFinWaves * ((size_t)M * 3 * A.kstride * sizeof(double2) + kMaxMol * 3 * sizeof(double));
   {
-    // several workgroups per placed list (as many as stay resident), so its
-    // insertions spread over more waves than one workgroup's
-    const int occ = occupancy(b, widom_finish_kernel, kFinWaves * 64, fin_lds);
+    // four insertions per wave where their tables fit, several workgroups per
+    // placed list (as many as stay resident), so its insertions spread over
+    // more waves than one workgroup's
+    const size_t lds4 = (size_t)kFinWaves * 4 * M * 3 * (A.kstride * sizeof(double2) + sizeof(double));
+    const bool four = M <= 4 && lds4 <= 64 * 1024;
+    const size_t lds = four ? lds4
+                            : (size_t)kFinWaves * ((size_t)M * 3 * A.kstride * sizeof(double2) + kMaxMol * 3 * sizeof(double));
+    void (*kern)(const WidomArgs) = widom_finish_any_kernel;
+    if (four) kern = M == 1 ? widom_finish_kernel<1> : (M == 2 ? widom_finish_kernel<2> : (M == 3 ? widom_finish_kernel<3> : widom_finish_kernel<4>));
+    const int occ = occupancy(b, kern, kFinWaves * 64, lds);
     const long long slots = (long long)std::max(1, occ) * std::max(1, b->n_cu);
     const int per = (int)std::max(1LL, std::min<long long>(kFinMaxPer, slots / A.groups));
-    rc = launch_ins(b, widom_finish_kernel, A, fin_lds, "widom_finish_kernel", kFinWaves, A.groups * per);
+    rc = launch_ins(b, kern, A, lds, "widom_finish_kernel", kFinWaves, A.groups * per);
   }
   if (rc) return rc;
   const int nblk = (n_insert + kRedBlock * kRedPer - 1) / (kRedBlock * kRedPer);
