@@ -111,6 +111,14 @@ struct graspa_box {
   int cell_n[3] = {0, 0, 0};
   int cell_cap = 0;
   int use_cells = 0;
+  // the framework in blocks of 16 neighbouring atoms for the pair kernel's
+  // block lists (WidomArgs), and whether it takes them
+  double2* d_fwb = nullptr;
+  int* d_fwb_type = nullptr;
+  float4* d_blk = nullptr;
+  int n_blk = 0, use_blocks = 0;
+  float blk_rcf = 0.0f;                // larger cutoff with the lists' margin
+  double blk_rmax = 0.0, blk_wmin = 0.0;   // largest half diagonal of a block, narrowest width of the cell
   // maps of the framework's certain-overlap volume per probe-site type
   // (dead_map.cpp), built on first use
   std::vector<uint32_t*> d_dmap;
@@ -273,6 +281,8 @@ __host__ __device__ inline double overlap_r2(double a4e, double s2, double shift
 
 // rows of the active k-vectors (engine_api.hip)
 int build_k_rows(graspa_box* b);
+// perpendicular widths of the cell along its three axes (engine_api.hip)
+void cell_widths(const graspa_box* b, double w[3]);
 // screen cell grid of the framework (engine_api.hip)
 int build_screen_cells(graspa_box* b);
 

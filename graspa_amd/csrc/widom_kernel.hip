@@ -63,6 +63,9 @@ constexpr int kFbWaves = 16;     // waves per workgroup of the first-bead kernel
 // g*chunk*cap_per_insertion; its length goes to counts[g].
 constexpr int kMaxScreenGroups = 1024;
 constexpr int kChainScreenMinAtoms = 4096;   // frameworks from this size screen orientation sites
+constexpr int kPairQueue = 128;        // pairs that a wave of it queues at most: under 64, and a step's
+constexpr int kGuestLds = 512;        // guest atoms that the list kernel keeps in LDS at most
+constexpr int kListCap = 256;          // block images a wave of the pair kernel lists at a time
 constexpr int kMaxTunePerCu = 8;       // workgroups per CU the autotuner tries at most
 constexpr int kMaxEvalGroups = 4096;   // workgroups of one pair-energy launch (work-count slots)
 
@@ -95,6 +98,17 @@ struct WidomArgs {
   int lj_general;               // the fast pair loop's general form: some LJ shift is nonzero, or a
                                 // molecule site's LJ with some framework type at r = 0.1 A stays
                                 // below twice OverlapCriteria (the r^2 < 0.01 test is then needed)
+  // the framework in blocks of 16 neighbouring atoms (and one of atoms at NaN),
+  // for the pair kernel's block lists
+  const double2* fwb;      // x,y and z,q [2][16 (n_blk + 1)]
+  const int* fwb_type;
+  const float4* blk;       // [2 n_blk] bounding boxes: centre in the cell, half edges
+  int n_blk;
+  float rcf;               // larger cutoff, rounded up
+  float list_reach;        // farthest site from the first bead (< 0: orientations list by site too)
+  int n_guest;             // guest atoms of all adsorbate components
+  int n_gl;                // entries of their LDS copy (0: read from memory)
+  int list_multi[2];       // by site / by insertion: a block may be in reach through two images on an axis
   int cell_n[3];
   int cell_cap;
   const uint4* ctab;       // [cells * cell_cap] fixed-point x,y,z + type, ~0u = empty
@@ -165,7 +179,7 @@ struct WidomArgs {
   unsigned long long* stat;   // screened pairs, evaluated pairs (sums of stat_part)
   // LDS layout (bytes from the start of the dynamic area)
   int lds_thr, lds_tab;                 // screening kernels
-  int lds_ffl, lds_coul, lds_fw;        // pair-energy kernel (lds_coul is 0)
+  int lds_ffl, lds_coul, lds_fw, lds_list, lds_q, lds_g;   // pair-energy kernel (lds_coul is 0)
 };
 
 // First insertion index of the batch.
@@ -574,6 +588,115 @@ __device__ inline int fw_type_slot(int i) { return ((i >> 7) << 7) + ((i & 63) <
 // bank, where 32-byte records put lanes l and l + 8 on the same banks).
 __device__ inline int fw_xy_slot(int i) { return ((i >> 7) << 8) + (((i >> 6) & 1) << 7) + (i & 63); }
 
+// Set-up of a pair-energy workgroup: exclusive prefix sums `pre` of the G
+// sub-lists' lengths, the force-field rows of the molecule's sites, and (fast
+// form) the real-space table, which sits at LDS offset 0 (lds_coul == 0), so
+// that a row's address is one multiply of its index.  The caller synchronizes.
+template <bool MIXED, int W>
+__device__ inline void eval_setup(const WidomArgs& A, const unsigned* counts, int G, unsigned* pre, double4* ffl,
+                                  double2* ct)
+{
+  for (int i = threadIdx.x; i < G; i += blockDim.x) pre[i + 1] = counts[i];
+  if (threadIdx.x == 0) pre[0] = 0u;
+  __syncthreads();
+  for (int h = 1; h < G; h <<= 1) {
+    unsigned add[(kMaxScreenGroups + W * 64 - 1) / (W * 64)];
+    for (int k = 0, i = threadIdx.x; i < G; ++k, i += blockDim.x) add[k] = (i >= h) ? pre[i + 1 - h] : 0u;
+    __syncthreads();
+    for (int k = 0, i = threadIdx.x; i < G; ++k, i += blockDim.x) pre[i + 1] += add[k];
+    __syncthreads();
+  }
+  const int T = A.bc.ntypes;
+  for (int i = threadIdx.x; i < A.M * T; i += blockDim.x) {
+    const int a = i / T, ty = i % T;
+    const double* f = A.ff64 + 4 * (ty * T + A.site_type[a]);
+    if (MIXED) {
+      // fast form: {c12, c6, shift} = {4 eps sigma^12, 4 eps sigma^6, shift}
+      const double s6 = f[1] * f[1] * f[1], c6 = f[0] * s6;
+      ffl[i] = make_double4(c6 * s6, c6, f[2], 0.0);
+    } else {
+      ffl[i] = make_double4(f[0], f[1], f[2], 0.0);
+    }
+  }
+  if (MIXED)
+    for (int i = threadIdx.x; i < A.coul_n / 2; i += blockDim.x)
+      ct[(i / (kCoulTabStride / 2)) * kCoulLdsRow + i % (kCoulTabStride / 2)] = reinterpret_cast<const double2*>(A.coul)[i];
+}
+
+// Sub-list holding point pi: the last lo with pre[lo] <= pi (from scratch, or
+// forward from the sub-list of an earlier point).
+__device__ inline int eval_sublist(const unsigned* pre, int G, int pi, int lo, bool search)
+{
+  if (search) {
+    int hi = G - 1;
+    lo = 0;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if ((int)pre[mid] <= pi) lo = mid; else hi = mid - 1;
+    }
+  }
+  while (lo + 1 < G && (int)pre[lo + 1] <= pi) ++lo;
+  return lo;
+}
+
+// Adds the pair of a trial site with one guest atom at (dx, dy, dz) from it,
+// of charge gq.
+template <bool MIXED, bool CUBIC>
+__device__ inline void guest_pair(const BoxConst& bc, const double2* ct, const double4* fr, bool coul, double sq, double dx,
+                                  double dy, double dz, double gq, int type, double& v, double& r, bool& o)
+{
+  if (MIXED)
+    pbc_rint<CUBIC>(dx, dy, dz, bc.cell, bc.inv);
+  else
+    pbc_fp64(dx, dy, dz, bc.cell, bc.inv, CUBIC ? 1 : 0);
+  const double rr = dx * dx + dy * dy + dz * dz;
+  if (rr < bc.cut_vdw2) {
+    const double4 ff = fr[type];
+    const double e = MIXED ? lj_mixed_c(rr, ff.x, ff.y, ff.z) : lj_fp64(rr, ff.x, ff.y, ff.z);
+    o = o || (e > bc.overlap) || (rr < 0.01);
+    v += e;
+  }
+  if (coul && rr < bc.cut_coul2) {
+    if (MIXED) {
+      r = fma(gq, coul_table(ct, rr), r);    // scaled with the framework's sum (eval_store)
+    } else {
+      const double rd = sqrt(rr);
+      r += bc.prefactor * 1.0 * (gq * sq * erfc(bc.alpha * rd)) / rd;
+    }
+  }
+}
+
+// Adds the pairs of one trial site with the guest molecules (guest-guest),
+// from memory.
+template <bool MIXED, bool CUBIC>
+__device__ inline void eval_guests(const WidomArgs& A, const double2* ct, const double4* fr, bool coul, double sq, double px,
+                                   double py, double pz, int lane, double& v, double& r, bool& o)
+{
+  for (int c = 1; c < A.gv.n_comp; ++c) {
+    const int ng = A.gv.seg[c].n_atoms, base = A.gv.seg[c].base;
+    for (int jj = lane; jj < ng; jj += 64) {
+      const int j = base + jj;
+      if (c == A.comp && A.g_molid[j] == A.new_molid) continue;
+      guest_pair<MIXED, CUBIC>(A.bc, ct, fr, coul, sq, A.g[j] - px, A.g[A.guest_cap + j] - py, A.g[2 * A.guest_cap + j] - pz,
+                               A.g[3 * A.guest_cap + j], A.g_type[j], v, r, o);
+    }
+  }
+}
+
+// Writes a trial site's sums: (LJ, real-space) energies and the overlap flag.
+template <bool MIXED>
+__device__ inline void eval_store(const WidomArgs& A, int slot, int ins, int bit, bool coul, double sq, int lane, double v,
+                                  double r, bool o, double2* energy, uint32_t* mask)
+{
+  const double sv = wave_sum(v);
+  const double sr = coul ? (MIXED ? (A.bc.prefactor * sq) * wave_sum(r) : wave_sum(r)) : 0.0;
+  const bool ov = __any(o) != 0;
+  if (lane == 0) {
+    energy[slot] = make_double2(sv, sr);
+    if (ov) atomicOr(mask + ins, 1u << bit);
+  }
+}
+
 // B / D: full energies of the trial sites of a work list (VDW_Coulomb.cu:
 // 1183-1352 for one trial site): wave sums of LJ and real-space Coulomb and
 // the exact overlap flag; one wave per site, 64 framework atoms per step.
@@ -587,40 +710,13 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 16 
   extern __shared__ __align__(16) char dyn[];
   __shared__ unsigned long long wg_eval;
   if (threadIdx.x == 0) wg_eval = 0ull;
-  // exclusive prefix sums of the sub-list lengths (groups sub-lists of
-  // chunk * per_ins entries each)
   __shared__ unsigned pre[kMaxScreenGroups + 1];
   const int G = groups;
-  for (int i = threadIdx.x; i < G; i += blockDim.x) pre[i + 1] = counts[i];
-  if (threadIdx.x == 0) pre[0] = 0u;
-  __syncthreads();
-  for (int h = 1; h < G; h <<= 1) {
-    unsigned add[(kMaxScreenGroups + W * 64 - 1) / (W * 64)];
-    for (int k = 0, i = threadIdx.x; i < G; ++k, i += blockDim.x) add[k] = (i >= h) ? pre[i + 1 - h] : 0u;
-    __syncthreads();
-    for (int k = 0, i = threadIdx.x; i < G; ++k, i += blockDim.x) pre[i + 1] += add[k];
-    __syncthreads();
-  }
+  double4* ffl = reinterpret_cast<double4*>(dyn + A.lds_ffl);
+  double2* ct = reinterpret_cast<double2*>(dyn);
+  eval_setup<MIXED, W>(A, counts, G, pre, ffl, ct);
   const BoxConst& bc = A.bc;
   const int T = bc.ntypes, n = A.n_fw;
-  double4* ffl = reinterpret_cast<double4*>(dyn + A.lds_ffl);
-  for (int i = threadIdx.x; i < A.M * T; i += blockDim.x) {
-    const int a = i / T, ty = i % T;
-    const double* f = A.ff64 + 4 * (ty * T + A.site_type[a]);
-    if (MIXED) {
-      // fast form: {c12, c6, shift} = {4 eps sigma^12, 4 eps sigma^6, shift}
-      const double s6 = f[1] * f[1] * f[1], c6 = f[0] * s6;
-      ffl[i] = make_double4(c6 * s6, c6, f[2], 0.0);
-    } else {
-      ffl[i] = make_double4(f[0], f[1], f[2], 0.0);
-    }
-  }
-  // the table sits at LDS offset 0 (lds_coul == 0): a row's address is one
-  // multiply of its index
-  double2* ct = reinterpret_cast<double2*>(dyn);
-  if (MIXED)
-    for (int i = threadIdx.x; i < A.coul_n / 2; i += blockDim.x)
-      ct[(i / (kCoulTabStride / 2)) * kCoulLdsRow + i % (kCoulTabStride / 2)] = reinterpret_cast<const double2*>(A.coul)[i];
   // the LDS copy is padded to whole steps of two atoms per lane with atoms at
   // NaN positions: every comparison with their r^2 is false, so they add
   // nothing, flag nothing and the steps need no bound check
@@ -656,16 +752,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 16 
   const int p_step = ranges ? 1 : nwave;
   int lo = 0;
   for (int pi = p_begin; pi < p_end; pi += p_step) {
-    if (!ranges || pi == p_begin) {
-      // sub-list g holding point pi: the last g with pre[g] <= pi
-      int hi = G - 1;
-      lo = 0;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if ((int)pre[mid] <= pi) lo = mid; else hi = mid - 1;
-      }
-    }
-    while (lo + 1 < G && (int)pre[lo + 1] <= pi) ++lo;
+    lo = eval_sublist(pre, G, pi, lo, !ranges || pi == p_begin);
     const TrialPt P = list[(size_t)lo * chunk * per_ins + (pi - (int)pre[lo])];
     const double px = P.x, py = P.y, pz = P.z;
     const double sq = A.site_q[P.site];
@@ -806,46 +893,285 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 16 
         }
       }
     }
-    // guest molecules (guest-guest), from memory
-    unsigned long long npair = (unsigned long long)n;
+    eval_guests<MIXED, CUBIC>(A, ct, fr, coul, sq, px, py, pz, lane, v, r, o);
+    n_eval += (unsigned long long)(n + A.n_guest);
+    eval_store<MIXED>(A, P.slot, P.ins, P.bit, coul, sq, lane, v, r, o, energy, mask);
+  }
+  if (lane == 0 && n_eval) atomicAdd(&wg_eval, n_eval);
+  __syncthreads();
+  if (threadIdx.x == 0) stat_slot[blockIdx.x] = wg_eval;
+}
+
+// The pair kernel of the FP64 form and of cells wider than the cutoff sphere
+// (use_blocks; the rule is at build_blocks).  A wave lists the images of the
+// framework's blocks of 16 neighbouring atoms within the cutoff of a centre
+// (64 blocks per step by their bounding boxes, in FP32 with a margin) and
+// visits only their atoms, a block per 16-lane row.  An atom is taken at the
+// image that its block is listed with, so a pair needs no minimum image; at
+// most one image of an atom is inside the cutoff.  About four in ten of the
+// visited pairs are inside it (a block is about 6 A wide): these go through a
+// queue in LDS to their energies, 64 at a time, so that no lane idles in the
+// long part (FP64 form: erfc and two divisions).  The centre is the site
+// itself for first beads; the orientations of an insertion share the list of
+// its first bead, longer by the molecule's reach.  A site's list, and with it
+// the order of its sums, is a function of its insertion alone.
+//
+// Both pair launches of 20,000 CO2 insertions, all atoms before and lists
+// now: 6,000 atoms in 48 A 2510 and 525 us (without the queue 577); 2,304 in
+// 40 x 40 x 27 A with 78 guest atoms 1620 and 1240 us (1340); 9,999 of N2,
+// 2,999 in a skewed 31 A cell, 1330 and 710 us (770).  Bound by the vector
+// units and LDS in about equal parts (20 instructions and 14 LDS cycles per
+// visited step, 40 and 60 per 64 energies).
+template <bool MIXED, bool CUBIC, bool FW_LDS, int W>
+__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 16 ? 8 : (MIXED && !FW_LDS && W == 12 ? 6 : 1)))) void widom_eval_list_kernel(
+    const WidomArgs A, const TrialPt* list, const unsigned* counts, int groups, int chunk, int per_ins, double2* energy,
+    uint32_t* mask, unsigned long long* stat_slot)
+{
+  extern __shared__ __align__(16) char dyn[];
+  __shared__ unsigned long long wg_eval;
+  if (threadIdx.x == 0) wg_eval = 0ull;
+  __shared__ unsigned pre[kMaxScreenGroups + 1];
+  const int G = groups;
+  double4* ffl = reinterpret_cast<double4*>(dyn + A.lds_ffl);
+  double2* ct = reinterpret_cast<double2*>(dyn);
+  eval_setup<MIXED, W>(A, counts, G, pre, ffl, ct);
+  const BoxConst& bc = A.bc;
+  const int T = bc.ntypes, npad = 16 * (A.n_blk + 1);
+  // lattice vectors n0 a + n1 b + n2 c of image code (n0 + 1) + 3 (n1 + 1) + 9 (n2 + 1)
+  double4* lat = reinterpret_cast<double4*>(dyn + A.lds_list);
+  if (threadIdx.x < 27) {
+    const int k = threadIdx.x;
+    const double n0 = k % 3 - 1, n1 = k / 3 % 3 - 1, n2 = k / 9 - 1;
+    lat[k] = make_double4(n0 * bc.cell[0] + n1 * bc.cell[3] + n2 * bc.cell[6],
+                          n0 * bc.cell[1] + n1 * bc.cell[4] + n2 * bc.cell[7],
+                          n0 * bc.cell[2] + n1 * bc.cell[5] + n2 * bc.cell[8], 0.0);
+  }
+  double2* fw2 = reinterpret_cast<double2*>(dyn + A.lds_fw);
+  int* fwt = reinterpret_cast<int*>(dyn + A.lds_fw + (size_t)npad * sizeof(double4));
+  if (FW_LDS)
+    for (int i = threadIdx.x; i < npad; i += blockDim.x) {
+      fw2[i] = A.fwb[i];
+      fw2[npad + i] = A.fwb[npad + i];
+      fwt[i] = A.fwb_type[i];
+    }
+  // the guest atoms, as many as n_gl says, without the inserted molecule's own
+  // slot; padded to whole wave steps with atoms at NaN
+  double2* gxy = reinterpret_cast<double2*>(dyn + A.lds_g);
+  double2* gzq = gxy + A.n_gl;
+  int* gty = reinterpret_cast<int*>(gzq + A.n_gl);
+  for (int i = threadIdx.x; i < A.n_gl; i += blockDim.x) {
+    const double nan = __builtin_nan("");
+    double2 xy = make_double2(nan, nan), zq = make_double2(nan, 0.0);
+    int ty = 0, k = i;
     for (int c = 1; c < A.gv.n_comp; ++c) {
-      const int ng = A.gv.seg[c].n_atoms, base = A.gv.seg[c].base;
-      npair += (unsigned long long)ng;
-      for (int jj = lane; jj < ng; jj += 64) {
-        const int j = base + jj;
-        if (c == A.comp && A.g_molid[j] == A.new_molid) continue;
-        const int ta = A.g_type[j];
-        const double gq = A.g[3 * A.guest_cap + j];
-        double dx = A.g[j] - px, dy = A.g[A.guest_cap + j] - py, dz = A.g[2 * A.guest_cap + j] - pz;
-        if (MIXED)
-          pbc_rint<CUBIC>(dx, dy, dz, bc.cell, bc.inv);
-        else
-          pbc_fp64(dx, dy, dz, bc.cell, bc.inv, CUBIC ? 1 : 0);
-        const double rr = dx * dx + dy * dy + dz * dz;
-        if (rr < bc.cut_vdw2) {
-          const double4 ff = fr[ta];
-          const double e = MIXED ? lj_mixed_c(rr, ff.x, ff.y, ff.z) : lj_fp64(rr, ff.x, ff.y, ff.z);
-          o = o || (e > bc.overlap) || (rr < 0.01);
-          v += e;
-        }
-        if (coul && rr < bc.cut_coul2) {
+      const int ng = A.gv.seg[c].n_atoms, j = A.gv.seg[c].base + k;
+      if (k >= 0 && k < ng && !(c == A.comp && A.g_molid[j] == A.new_molid)) {
+        xy = make_double2(A.g[j], A.g[A.guest_cap + j]);
+        zq = make_double2(A.g[2 * A.guest_cap + j], A.g[3 * A.guest_cap + j]);
+        ty = A.g_type[j];
+      }
+      k -= ng;
+    }
+    gxy[i] = xy; gzq[i] = zq; gty[i] = ty;
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = lane >> 4, at = lane & 15;
+  unsigned* lst = reinterpret_cast<unsigned*>(dyn + A.lds_list + 27 * sizeof(double4)) + wv * kListCap;
+  // the wave's queue of pairs inside the cutoff: (r^2, charge) and type
+  double2* qa = reinterpret_cast<double2*>(dyn + A.lds_q) + wv * kPairQueue;
+  int* qt = reinterpret_cast<int*>(dyn + A.lds_q + (size_t)W * kPairQueue * sizeof(double2)) + wv * kPairQueue;
+  const bool orient = list == A.list2;
+  const bool by_ins = orient && A.list_reach >= 0.0f;     // else by site
+  const float R = A.rcf + (by_ins ? A.list_reach : 0.0f), R2 = R * R;
+  const int lg = A.list_multi[by_ins ? 1 : 0] ? 3 : 0, n_step = (A.n_blk + 63) >> 6 << lg;
+  const bool same = bc.cut_vdw2 == bc.cut_coul2;
+  const int npts = __builtin_amdgcn_readfirstlane((int)pre[G]);
+  unsigned long long n_eval = 0;
+  // points to waves as in widom_eval_kernel
+  const int nwave = gridDim.x * W, wid = blockIdx.x * W + wv;
+  const int per_wave = (npts + nwave - 1) / nwave;
+  const bool ranges = per_wave >= 4;
+  const int p_begin = ranges ? wid * per_wave : wid, p_end = ranges ? min(npts, p_begin + per_wave) : npts;
+  const size_t stride = (size_t)chunk * per_ins;
+  int lo = 0, nit = 0, have = -1;      // `have`: the insertion whose whole list is in lst, of nit steps
+  for (int pi = p_begin; pi < p_end; pi += ranges ? 1 : nwave) {
+    lo = __builtin_amdgcn_readfirstlane(eval_sublist(pre, G, pi, lo, !ranges || pi == p_begin));
+    const TrialPt P = list[lo * stride + (pi - (int)pre[lo])];
+    // the centre, moved into the cell, and the site with it (all wave-uniform)
+    const int ins = __builtin_amdgcn_readfirstlane(P.ins), site = __builtin_amdgcn_readfirstlane(P.site);
+    const int slot = __builtin_amdgcn_readfirstlane(P.slot), bit = __builtin_amdgcn_readfirstlane(P.bit);
+    double c0 = P.x, c1 = P.y, c2 = P.z;
+    if (by_ins) {
+      const double* fb = A.state[ins].fb;
+      c0 = fb[0]; c1 = fb[1]; c2 = fb[2];
+    }
+    const double w0 = -floor(bc.inv[0] * c0 + bc.inv[3] * c1 + bc.inv[6] * c2);
+    const double w1 = -floor(bc.inv[1] * c0 + bc.inv[4] * c1 + bc.inv[7] * c2);
+    const double w2 = -floor(bc.inv[2] * c0 + bc.inv[5] * c1 + bc.inv[8] * c2);
+    auto into = [&](double x, int d) {
+      return readlane_d(fma(w0, bc.cell[d], fma(w1, bc.cell[3 + d], fma(w2, bc.cell[6 + d], x))), 0);
+    };
+    const double sx = into(P.x, 0), sy = into(P.y, 1), sz = into(P.z, 2), sq = A.site_q[site];
+    const bool coul = bc.use_charges && sq != 0.0;
+    const double4* fr = ffl + site * T;
+    double v = 0.0, r = 0.0;
+    bool o = false;
+    const double cut2 = coul ? fmax(bc.cut_vdw2, bc.cut_coul2) : bc.cut_vdw2;
+    const float fx = (float)(by_ins ? into(c0, 0) : sx), fy = (float)(by_ins ? into(c1, 1) : sy);
+    const float fz = (float)(by_ins ? into(c2, 2) : sz);
+    int qn = 0;      // pairs in the queue, under 64 between steps
+    // the energies of the queue's last m pairs, one per lane
+    auto drain = [&](auto same_c, auto general_c, int m) {
+      constexpr bool SAME = decltype(same_c)::value;        // equal LJ and Coulomb cutoffs
+      constexpr bool GENERAL = decltype(general_c)::value;  // as in widom_eval_kernel
+      wave_sync();
+      qn -= m;
+      if (lane < m) {
+        const double2 rq = qa[qn + lane];
+        const double rr = rq.x;
+        const double4* f = fr + qt[qn + lane];
+        const double2 cc = *reinterpret_cast<const double2*>(f);
+        if (SAME || rr < bc.cut_vdw2) {
           if (MIXED) {
-            r = fma(gq, coul_table(ct, rr), r);    // scaled with the framework sum below
+            const double en = lj_mixed_c(rr, cc.x, cc.y, GENERAL ? f->z : 0.0);
+            v += en;
+            o = o || !(en <= bc.overlap) || (GENERAL && rr < 0.01);
+          } else {
+            const double en = lj_fp64(rr, cc.x, cc.y, f->z);
+            o = o || (en > bc.overlap) || (rr < 0.01);
+            v += en;
+          }
+        }
+        if (coul && (SAME || rr < bc.cut_coul2)) {
+          if (MIXED) {
+            r = fma(rq.y, coul_table(ct, rr), r);
           } else {
             const double rd = sqrt(rr);
-            r += bc.prefactor * 1.0 * (gq * sq * erfc(bc.alpha * rd)) / rd;
+            r += bc.prefactor * 1.0 * (rq.y * sq * erfc(bc.alpha * rd)) / rd;
           }
         }
       }
+      wave_sync();
+    };
+    // the listed blocks' atoms, one per lane and step, the next step's read
+    // while this one's are used; those inside the cutoff join the queue, so
+    // that the energies run with full waves
+    auto visit = [&](auto same_c, auto general_c, bool end) {
+      struct Atom {
+        double2 xy, zq;
+        int ty;
+        unsigned img;
+      };
+      auto read = [&](int it) {
+        const unsigned e = lst[4 * it + row];
+        Atom a;
+        a.img = e & 31u;
+        if (FW_LDS) {
+          const int j = (int)(e >> 5) * 16 + at;
+          a.xy = fw2[j]; a.zq = fw2[npad + j]; a.ty = fwt[j];
+        } else {
+          // (byte offsets below 4 GB: one 32-bit offset to a scalar base)
+          const unsigned k = ((e & ~31u) << 3) | (unsigned)(at << 4);
+          a.xy = *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(A.fwb) + k);
+          a.zq = *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(A.fwb + npad) + k);
+          a.ty = *reinterpret_cast<const int*>(reinterpret_cast<const char*>(A.fwb_type) + (k >> 2));
+        }
+        return a;
+      };
+      auto add = [&](const Atom& a) {
+        const double4 sh = lat[a.img];
+        const double dx = a.xy.x + sh.x - sx, dy = a.xy.y + sh.y - sy, dz = a.zq.x + sh.z - sz;
+        const double rr = fma(dz, dz, fma(dy, dy, dx * dx));
+        const bool in = rr < cut2;
+        const unsigned long long im = __ballot(in);
+        if (!im) return;
+        const int pos = qn + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(im >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((unsigned)im, 0u));
+        if (in) {
+          qa[pos] = make_double2(rr, a.zq.y);
+          qt[pos] = a.ty;
+        }
+        qn += __popcll(im);
+        if (qn >= 64) drain(same_c, general_c, 64);
+      };
+      if (nit > 0) {
+        // (the two steps of a pass read into each other's registers)
+        Atom a0 = read(0);
+        for (int it = 0;;) {
+          const Atom a1 = read(min(it + 1, nit - 1));
+          add(a0);
+          if (++it >= nit) break;
+          a0 = read(min(it + 1, nit - 1));
+          add(a1);
+          if (++it >= nit) break;
+        }
+      }
+      if (end && qn > 0) drain(same_c, general_c, qn);
+    };
+    const bool listed = by_ins && ins == have;
+    int step = listed ? n_step : 0;
+    bool whole = true;
+    for (;;) {
+      if (step < n_step) {
+        int cnt = 0;
+        for (; step < n_step && cnt <= kListCap - 68; ++step) {
+          // steps of 64 blocks, for each of their images if there may be more than one
+          const int k = step & ((1 << lg) - 1), blk = (step >> lg) * 64 + lane;
+          const bool in = blk < A.n_blk;
+          const float4 B = A.blk[2 * (in ? blk : 0)], H = A.blk[2 * (in ? blk : 0) + 1];
+          const float ex = B.x - fx, ey = B.y - fy, ez = B.z - fz;
+          float f0 = (float)bc.inv[0] * ex, f1 = (float)bc.inv[4] * ey, f2 = (float)bc.inv[8] * ez;
+          if (!CUBIC) {
+            f0 += (float)bc.inv[3] * ey + (float)bc.inv[6] * ez;
+            f1 += (float)bc.inv[1] * ex + (float)bc.inv[7] * ez;
+            f2 += (float)bc.inv[2] * ex + (float)bc.inv[5] * ey;
+          }
+          // on each axis the nearest image of the block's centre, or (bits of
+          // k) the one a period further, on the other side: no other is in reach
+          float m0 = -rintf(f0), m1 = -rintf(f1), m2 = -rintf(f2);
+          if (k & 1) m0 += f0 + m0 < 0.0f ? 1.0f : -1.0f;
+          if (k & 2) m1 += f1 + m1 < 0.0f ? 1.0f : -1.0f;
+          if (k & 4) m2 += f2 + m2 < 0.0f ? 1.0f : -1.0f;
+          float qx = fmaf(m0, (float)bc.cell[0], ex), qy = fmaf(m1, (float)bc.cell[4], ey);
+          float qz = fmaf(m2, (float)bc.cell[8], ez);
+          if (!CUBIC) {
+            qx += m1 * (float)bc.cell[3] + m2 * (float)bc.cell[6];
+            qy += m0 * (float)bc.cell[1] + m2 * (float)bc.cell[7];
+            qz += m0 * (float)bc.cell[2] + m1 * (float)bc.cell[5];
+          }
+          qx = fmaxf(fabsf(qx) - H.x, 0.0f); qy = fmaxf(fabsf(qy) - H.y, 0.0f); qz = fmaxf(fabsf(qz) - H.z, 0.0f);
+          // (both centres are in the cell, so |m| <= 1 unless rounding put
+          // them a whole period apart: out of reach)
+          const bool hit = in && fmaf(qz, qz, fmaf(qy, qy, qx * qx)) < R2 && fabsf(m0) <= 1.0f && fabsf(m1) <= 1.0f &&
+                           fabsf(m2) <= 1.0f;
+          const unsigned long long hm = __ballot(hit);
+          const int pos = cnt + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(hm >> 32),
+                                                               __builtin_amdgcn_mbcnt_lo((unsigned)hm, 0u));
+          if (hit) lst[pos] = ((unsigned)blk << 5) | (unsigned)((int)m0 + 3 * (int)m1 + 9 * (int)m2 + 13);
+          cnt += __popcll(hm);
+        }
+        nit = (cnt + 3) >> 2;
+        if (lane < 4 * nit - cnt) lst[cnt + lane] = (unsigned)A.n_blk << 5;     // (the block of atoms at NaN)
+        whole = whole && step == n_step;
+        wave_sync();
+      }
+      const bool end = step >= n_step;
+      if (MIXED && A.lj_general) visit(std::false_type{}, std::true_type{}, end);   // (equal cutoffs or not)
+      else if (same) visit(std::true_type{}, std::false_type{}, end);
+      else visit(std::false_type{}, std::false_type{}, end);
+      wave_sync();
+      if (step >= n_step) break;
     }
-    n_eval += npair;
-    const double sv = wave_sum(v);
-    const double sr = coul ? (MIXED ? (bc.prefactor * sq) * wave_sum(r) : wave_sum(r)) : 0.0;
-    const bool ov = __any(o) != 0;
-    if (lane == 0) {
-      energy[P.slot] = make_double2(sv, sr);
-      if (ov) atomicOr(mask + P.ins, 1u << P.bit);
+    have = by_ins && whole ? ins : -1;
+    // guest molecules (guest-guest)
+    for (int j = lane; j < A.n_gl; j += 64) {
+      const double2 xy = gxy[j], zq = gzq[j];
+      guest_pair<MIXED, CUBIC>(bc, ct, fr, coul, sq, xy.x - sx, xy.y - sy, zq.x - sz, zq.y, gty[j], v, r, o);
     }
+    if (A.n_gl == 0) eval_guests<MIXED, CUBIC>(A, ct, fr, coul, sq, sx, sy, sz, lane, v, r, o);
+    n_eval += (unsigned long long)(A.n_fw + A.n_guest);
+    eval_store<MIXED>(A, slot, ins, bit, coul, sq, lane, v, r, o, energy, mask);
   }
   if (lane == 0 && n_eval) atomicAdd(&wg_eval, n_eval);
   __syncthreads();
@@ -1559,25 +1885,33 @@ static int ensure_pipeline(graspa_box* b, int n_insert, int K, int OC)
 using EvalKern = void (*)(const WidomArgs, const TrialPt*, const unsigned*, int, int, int, double2*, uint32_t*,
                           unsigned long long*);
 
-template <bool MIXED, bool CUBIC, bool FW_LDS>
+template <bool MIXED, bool CUBIC, bool FW_LDS, bool LIST>
 static EvalKern eval_kernel_w(int waves)
 {
   switch (waves) {
-    case 4: return widom_eval_kernel<MIXED, CUBIC, FW_LDS, 4>;
-    case 8: return widom_eval_kernel<MIXED, CUBIC, FW_LDS, 8>;
-    case 16: return widom_eval_kernel<MIXED, CUBIC, FW_LDS, 16>;
-    default: return widom_eval_kernel<MIXED, CUBIC, FW_LDS, 12>;
+    case 4: return LIST ? widom_eval_list_kernel<MIXED, CUBIC, FW_LDS, 4> : widom_eval_kernel<MIXED, CUBIC, FW_LDS, 4>;
+    case 8: return LIST ? widom_eval_list_kernel<MIXED, CUBIC, FW_LDS, 8> : widom_eval_kernel<MIXED, CUBIC, FW_LDS, 8>;
+    case 16: return LIST ? widom_eval_list_kernel<MIXED, CUBIC, FW_LDS, 16> : widom_eval_kernel<MIXED, CUBIC, FW_LDS, 16>;
+    default: return LIST ? widom_eval_list_kernel<MIXED, CUBIC, FW_LDS, 12> : widom_eval_kernel<MIXED, CUBIC, FW_LDS, 12>;
   }
 }
 
 // The pair-energy kernel of a launch shape for the box's precision form and cell.
-static EvalKern eval_kernel_for(const graspa_box* b, int waves, bool fw_lds)
+template <bool LIST>
+static EvalKern eval_kernel_l(const graspa_box* b, int waves, bool fw_lds)
 {
   const bool mixed = b->precision == GRASPA_MIXED, cubic = b->bc.cubic != 0;
-  if (mixed && cubic) return fw_lds ? eval_kernel_w<true, true, true>(waves) : eval_kernel_w<true, true, false>(waves);
-  if (mixed) return fw_lds ? eval_kernel_w<true, false, true>(waves) : eval_kernel_w<true, false, false>(waves);
-  if (cubic) return fw_lds ? eval_kernel_w<false, true, true>(waves) : eval_kernel_w<false, true, false>(waves);
-  return fw_lds ? eval_kernel_w<false, false, true>(waves) : eval_kernel_w<false, false, false>(waves);
+  if (mixed && cubic)
+    return fw_lds ? eval_kernel_w<true, true, true, LIST>(waves) : eval_kernel_w<true, true, false, LIST>(waves);
+  if (mixed)
+    return fw_lds ? eval_kernel_w<true, false, true, LIST>(waves) : eval_kernel_w<true, false, false, LIST>(waves);
+  if (cubic)
+    return fw_lds ? eval_kernel_w<false, true, true, LIST>(waves) : eval_kernel_w<false, true, false, LIST>(waves);
+  return fw_lds ? eval_kernel_w<false, false, true, LIST>(waves) : eval_kernel_w<false, false, false, LIST>(waves);
+}
+static EvalKern eval_kernel_for(const graspa_box* b, int waves, bool fw_lds)
+{
+  return b->use_blocks ? eval_kernel_l<true>(b, waves, fw_lds) : eval_kernel_l<false>(b, waves, fw_lds);
 }
 
 // LDS of the pair-energy kernel before the framework: FF rows of the species'
@@ -1591,9 +1925,33 @@ static size_t eval_lds_base(const graspa_box* b, int M)
   return align16(eval_lds_coul_bytes(b) + (size_t)M * b->bc.ntypes * sizeof(double4));
 }
 
-static size_t eval_lds(const graspa_box* b, size_t base, bool fw_lds)
+// Guest atoms, and the entries of the list kernel's LDS copy of them: whole
+// wave steps, none if they are more than kGuestLds (read from memory then).
+static int guest_atoms(const graspa_box* b)
 {
-  return base + (fw_lds ? align16((size_t)eval_fw_pad(b->n_fw) * (sizeof(double4) + sizeof(int))) : 0);
+  GuestView gv;
+  guest_view(b, &gv);
+  int n = 0;
+  for (int c = 1; c < gv.n_comp; ++c) n += gv.seg[c].n_atoms;
+  return n;
+}
+static int guest_lds_entries(const graspa_box* b)
+{
+  const int n = (guest_atoms(b) + 63) / 64 * 64;
+  return b->use_blocks && n <= kGuestLds ? n : 0;
+}
+// Bytes of the block lists: the lattice vectors, a list per wave, the guests.
+static size_t eval_lds_list(const graspa_box* b, int waves)
+{
+  if (!b->use_blocks) return 0;
+  return 27 * sizeof(double4) + (size_t)waves * kListCap * sizeof(unsigned) +
+         (size_t)waves * kPairQueue * (sizeof(double2) + sizeof(int)) +
+         align16((size_t)guest_lds_entries(b) * (sizeof(double4) + sizeof(int)));
+}
+static size_t eval_lds(const graspa_box* b, size_t base, int waves, bool fw_lds)
+{
+  const size_t n = b->use_blocks ? 16 * (size_t)(b->n_blk + 1) : (size_t)eval_fw_pad(b->n_fw);
+  return base + eval_lds_list(b, waves) + (fw_lds ? align16(n * (sizeof(double4) + sizeof(int))) : 0);
 }
 
 // Grid of one pair-energy launch: per_cu workgroups per CU (0: as many as
@@ -1616,7 +1974,11 @@ static int launch_eval(graspa_box* b, const WidomArgs& A, const TrialPt* list, c
   const int waves = b->ev_waves;
   for (int pass = b->ev_fw_lds ? 0 : 1; pass < 2; ++pass) {
     const bool fw_lds = pass == 0;
-    const size_t lds = eval_lds(b, (size_t)A.lds_fw, fw_lds);
+    const size_t lds = eval_lds(b, (size_t)A.lds_list, waves, fw_lds);
+    // the list kernel as its default shape: the framework in LDS only where
+    // two workgroups share a CU: 12 waves with it in LDS take 1587 us of the
+    // loaded box's batch, 24 that read it through the caches 1268
+    if (b->use_blocks && fw_lds && b->ev_per_cu == 0 && lds > 80 * 1024) continue;
     const EvalKern kern = eval_kernel_for(b, waves, fw_lds);
     const int grid = eval_grid(b, kern, waves, lds, b->ev_per_cu);
     if (grid < 1) continue;
@@ -1918,10 +2280,28 @@ int launch_widom(graspa_box* b, int comp, int K, int O, double beta, int bias, d
   A.lds_tab = (int)scr_base;
   const size_t tab_bytes =
       A.use_cells ? (size_t)b->cell_n[0] * b->cell_n[1] * b->cell_n[2] * b->cell_cap * sizeof(uint4) : 0;
-  // pair-energy kernel: Coulomb table (fast form) | FF rows | framework (optional)
+  // pair-energy kernel: Coulomb table (fast form) | FF rows | block lists | framework (optional)
   A.lds_coul = 0;
   A.lds_ffl = (int)eval_lds_coul_bytes(b);
-  A.lds_fw = (int)eval_lds_base(b, M);
+  A.lds_list = (int)eval_lds_base(b, M);
+  A.lds_fw = A.lds_list + (int)eval_lds_list(b, b->ev_waves);
+  A.fwb = b->d_fwb; A.fwb_type = b->d_fwb_type; A.blk = b->d_blk; A.n_blk = b->n_blk;
+  A.rcf = b->blk_rcf;
+  A.n_guest = guest_atoms(b);
+  A.n_gl = guest_lds_entries(b);
+  A.lds_q = A.lds_list + (int)(27 * sizeof(double4) + (size_t)b->ev_waves * kListCap * sizeof(unsigned));
+  A.lds_g = A.lds_q + (int)((size_t)b->ev_waves * kPairQueue * (sizeof(double2) + sizeof(int)));
+  A.list_reach = -1.0f;
+  A.list_multi[0] = A.list_multi[1] = 0;
+  if (b->use_blocks) {
+    double d2 = 0.0;
+    for (int a = 0; a < A.chain; ++a)
+      d2 = std::max(d2, A.tvec[a][0] * A.tvec[a][0] + A.tvec[a][1] * A.tvec[a][1] + A.tvec[a][2] * A.tvec[a][2]);
+    const double d = std::sqrt(d2) * (1.0 + 1e-6) + 1e-3, far = b->blk_rcf + b->blk_rmax;
+    if (far + d < 0.99 * b->blk_wmin) A.list_reach = (float)d;
+    A.list_multi[0] = far > 0.5 * b->blk_wmin;
+    A.list_multi[1] = far + d > 0.5 * b->blk_wmin;
+  }
   const bool cubic = A.bc.cubic != 0;
   if (how.key) {
     const unsigned char* a = reinterpret_cast<const unsigned char*>(&A);
@@ -2010,7 +2390,7 @@ int widom_autotune(graspa_box* b, int comp, int K, int O, double beta, int bias,
   std::vector<graspa_eval_shape> cand;
   for (const int w : {4, 8, 12, 16})
     for (int f = 1; f >= 0; --f) {
-      const int occ = occupancy(b, eval_kernel_for(b, w, f != 0), w * 64, eval_lds(b, base, f != 0));
+      const int occ = occupancy(b, eval_kernel_for(b, w, f != 0), w * 64, eval_lds(b, base, w, f != 0));
       for (int p = 1; p <= std::min(occ, kMaxTunePerCu); ++p) cand.push_back(graspa_eval_shape{w, p, f});
     }
   if (cand.empty()) return fail(GRASPA_ERR_UNSUPPORTED, "widom: no launch shape fits the LDS (pair energies)");
