@@ -56,6 +56,7 @@ constexpr int kBGroup = 8;             // sites per pass over the atoms
 // framework atoms and one of the guest atoms within the pass's reach
 constexpr int kLocFw = 256;            // framework entries per wave
 constexpr int kLocG = 128;             // guest entries per wave
+constexpr int kPairQueue = 128;        // FP64 form: pairs that a wave queues at most (under 64, and a step's)
 constexpr int kBDrawTrial = 16;        // first trial draw
 constexpr int kBMaxDraws = kBDrawTrial + 9 * kBMaxTrial;   // K trials, O orientations, O retrace orientations
 
@@ -179,6 +180,7 @@ struct BMove {
   // per-wave entry counts (framework, guests) and their prefix sums
   double lc[3], lr2;
   int loc_on, loc_over;
+  int queue;                         // FP64 form: the pair queues are there (behind the list segments)
   int lcnt[2][kBW], lpre[2][kBW + 1];
 };
 
@@ -335,6 +337,144 @@ __device__ void block_sums(const BBox& B, const BState& S, const int bk, const i
   if (t == 0) st.cycles[bk] += 1;
 }
 
+// The FP64 form's part of a pair pass: a wave's atoms (every stride-th 64 from
+// k0 on) against the sites [g0, g0 + cnt) of its group; the sums go to
+// L.part, the result is the overlap mask (bit site - g0).  The pairs inside
+// the cutoff go through a queue in LDS, so that erfc, the square root and the
+// divisions run 64 pairs at a time whatever sites they belong to: about a
+// sixth of the pairs of a 40 x 40 x 27 A box are inside, in nearly every wave
+// step of some site (10 cycles of that box, 2,304 atoms, 26 CO2 and more:
+// 30.3 and 25.3 ms).  Without room for the queues in LDS the pass runs as the
+// fast form's, whose pairs are a third as long.
+template <bool CUBIC>
+__device__ uint32_t pair_queue(const BBox& B, const BState& S, BMove& L, const double* __restrict__ ffl,
+                               const double* __restrict__ fwl, const double* __restrict__ gml, int* __restrict__ loc,
+                               const bool use_loc, const int g0, const int cnt, const int k0, const int stride,
+                               const int ex_lo, const int ex_hi)
+{
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const BoxConst& bc = B.bc;
+  const int T = bc.ntypes, nf = B.n_fw, cap = B.guest_cap;
+  double* q_rr = reinterpret_cast<double*>(loc + kBW * (kLocFw + kLocG)) + wave * 2 * kPairQueue;
+  double* q_q = q_rr + kPairQueue;
+  int* q_t = reinterpret_cast<int*>(reinterpret_cast<double*>(loc + kBW * (kLocFw + kLocG)) + kBW * 2 * kPairQueue) +
+             wave * kPairQueue;
+  const double cut2 = bc.use_charges ? fmax(bc.cut_vdw2, bc.cut_coul2) : bc.cut_vdw2;
+  uint32_t ovb = 0;
+#pragma unroll 1
+  for (int part = 0; part < 2; ++part) {
+    double av[kBGroup], ar[kBGroup];
+#pragma unroll
+    for (int j = 0; j < kBGroup; ++j) { av[j] = 0.0; ar[j] = 0.0; }
+    // atoms of the part: the neighbour list's, or all
+    int n = 0;
+    if (use_loc) n = L.lpre[part][kBW];
+    else if (part == 0) n = nf;
+    else
+      for (int c = 1; c < B.n_comp; ++c) n += S.n_mol[c] * B.sp[c].molsize;
+    int qn = 0;
+    // steps over the atoms, and a last one that empties the queue
+#pragma unroll 1
+    for (int kb = k0; ; kb += stride) {
+      const bool last = kb >= n;
+      double ax = 0.0, ay = 0.0, az = 0.0, aq = 0.0;
+      int at = 0;
+      const int k = kb + lane;
+      bool have = k < n;
+      if (have) {
+        int i = k;
+        if (use_loc) {
+          const int* pre = L.lpre[part];
+          int w = 0;
+          while (w + 1 < kBW && pre[w + 1] <= k) ++w;
+          i = loc[(part == 0 ? w * kLocFw : kBW * kLocFw + w * kLocG) + (k - pre[w])];
+        }
+        if (part == 0) {
+          if (fwl) {
+            ax = fwl[i]; ay = fwl[nf + i]; az = fwl[2 * nf + i]; aq = fwl[3 * nf + i];
+            at = reinterpret_cast<const int*>(fwl + 4 * nf)[i];
+          } else {
+            ax = B.fw[i]; ay = B.fw[nf + i]; az = B.fw[2 * nf + i]; aq = B.fw[3 * nf + i]; at = B.fw_type[i];
+          }
+        } else {
+          // the guest's species: by its slot in the store, or by its rank
+          int c = 1;
+          if (use_loc) {
+            while (c + 1 < B.n_comp && i >= B.sp[c + 1].base) ++c;
+          } else {
+            while (c + 1 < B.n_comp && i >= S.n_mol[c] * B.sp[c].molsize) { i -= S.n_mol[c] * B.sp[c].molsize; ++c; }
+            i += B.sp[c].base;
+          }
+          have = !(i >= ex_lo && i < ex_hi);
+          if (have) {
+            const int gn = L.gl_n, m = i - B.sp[c].base + L.gl_off[c];
+            if (gml && S.n_mol[c] * B.sp[c].molsize <= L.gl_cap[c]) {
+              ax = gml[m]; ay = gml[gn + m]; az = gml[2 * gn + m]; aq = gml[3 * gn + m];
+              at = reinterpret_cast<const int*>(gml + 4 * gn)[m];
+            } else {
+              ax = B.g[i]; ay = B.g[cap + i]; az = B.g[2 * cap + i]; aq = B.g[3 * cap + i]; at = B.g_type[i];
+            }
+          }
+        }
+      }
+#pragma unroll 1
+      for (int j = 0; j < (last ? 1 : cnt); ++j) {
+        if (!last) {
+          const BSite& s = L.site[L.idx[g0 + j]];
+          double dx = ax - s.x, dy = ay - s.y, dz = az - s.z;
+          pbc_fp64(dx, dy, dz, bc.cell, bc.inv, CUBIC ? 1 : 0);
+          const double rr = dx * dx + dy * dy + dz * dz;
+          const bool in = have && rr < cut2;
+          const unsigned long long im = __ballot(in);
+          if (im) {
+            const int pos = qn + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(im >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((unsigned)im, 0u));
+            if (in) {
+              q_rr[pos] = rr;
+              q_q[pos] = aq;
+              q_t[pos] = at | (j << 16);
+            }
+            qn += __popcll(im);
+          }
+        }
+        const int m = last ? qn : (qn >= 64 ? 64 : 0);
+        if (m > 0) {
+          // the queue's last m pairs, one per lane
+          wave_sync();
+          qn -= m;
+          double ev = 0.0, er = 0.0;
+          int tag = -1;
+          if (lane < m) {
+            const double rr = q_rr[qn + lane], q = q_q[qn + lane];
+            const int ty = q_t[qn + lane] & 0xffff;
+            tag = q_t[qn + lane] >> 16;
+            const BSite& s = L.site[L.idx[g0 + tag]];
+            if (rr < bc.cut_vdw2) {
+              const double* f = ffl + 4 * (ty * T + s.type);
+              ev = lj_fp64(rr, f[0], f[1], f[2]);
+              if (ev > bc.overlap || rr < 0.01) ovb |= 1u << tag;
+            }
+            if (bc.use_charges && rr < bc.cut_coul2) {
+              const double d = sqrt(rr);
+              const double term = q * s.q * erfc(bc.alpha * d);
+              er = bc.prefactor * 1.0 * term / d;
+            }
+          }
+#pragma unroll
+          for (int g = 0; g < kBGroup; ++g) {
+            av[g] += tag == g ? ev : 0.0;
+            ar[g] += tag == g ? er : 0.0;
+          }
+          wave_sync();
+        }
+      }
+      if (last) break;
+    }
+    wave_sum_group(av, ar, L.part[part][wave]);
+  }
+  return ovb;
+}
+
 template <bool MIXED, bool CUBIC>
 __device__ void pair_pass(const BBox& B, const BState& S, BMove& L, const double* __restrict__ ffl,
                           const double2* __restrict__ ct, const double* __restrict__ fwl,
@@ -444,6 +584,9 @@ __device__ void pair_pass(const BBox& B, const BState& S, BMove& L, const double
   const int first = r * 64 + lane, stride = (w1 - w0) * 64;
   const int nf = B.n_fw, cap = B.guest_cap;
   uint32_t ovb = 0;
+  if (!MIXED && loc && L.queue) {
+    ovb = pair_queue<CUBIC>(B, S, L, ffl, fwl, gml, loc, use_loc, g0, cnt, r * 64, stride, ex_lo, ex_hi);
+  } else
 #pragma unroll 1
   for (int part = 0; part < 2; ++part) {
     double av[kBGroup], ar[kBGroup];
@@ -1683,10 +1826,12 @@ __global__ __launch_bounds__(kBT) void batch_mc_kernel(const BBox* __restrict__ 
   // then the pair passes' neighbour-list segments (cubic cells), then the
   // guest mirror
   const int l_off = fw_in_lds ? fw_off + 4 * nf + (nf + 1) / 2 : fw_off;
-  constexpr int kLocDoubles = kBW * (kLocFw + kLocG) / 2;
-  int* loc = (CUBIC && (size_t)(l_off + kLocDoubles) * 8 <= (size_t)dyn_bytes) ? reinterpret_cast<int*>(dyn + l_off)
-                                                                               : nullptr;
-  const int g_off = loc ? l_off + kLocDoubles : l_off;
+  // (FP64 form: with the pair queues behind the segments if both fit)
+  constexpr int kLocDoubles = kBW * (kLocFw + kLocG) / 2, kQueueDoubles = kBW * kPairQueue * 5 / 2;
+  const bool queue = !MIXED && (size_t)(l_off + kLocDoubles + kQueueDoubles) * 8 <= (size_t)dyn_bytes;
+  int* loc = (queue || (CUBIC && (size_t)(l_off + kLocDoubles) * 8 <= (size_t)dyn_bytes))
+                 ? reinterpret_cast<int*>(dyn + l_off) : nullptr;
+  const int g_off = loc ? l_off + kLocDoubles + (queue ? kQueueDoubles : 0) : l_off;
   const int g_room = dyn_bytes / 8 > g_off ? (int)((dyn_bytes / 8 - g_off) * 8 / 36) : 0;
   if (tid == 0) {
     const int ns = B.n_comp - 1, share = ns > 0 ? g_room / ns : 0;
@@ -1702,6 +1847,7 @@ __global__ __launch_bounds__(kBT) void batch_mc_kernel(const BBox* __restrict__ 
       n += cp;
     }
     L.gl_n = n;
+    L.queue = queue ? 1 : 0;
   }
   __syncthreads();
   double* gml = L.gl_n > 0 ? dyn + g_off : nullptr;

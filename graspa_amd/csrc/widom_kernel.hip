@@ -955,14 +955,13 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 16 
       fwt[i] = A.fwb_type[i];
     }
   // the guest atoms, as many as n_gl says, without the inserted molecule's own
-  // slot; padded to whole wave steps with atoms at NaN
+  // slot; padded to whole wave steps with entries of type -1
   double2* gxy = reinterpret_cast<double2*>(dyn + A.lds_g);
   double2* gzq = gxy + A.n_gl;
   int* gty = reinterpret_cast<int*>(gzq + A.n_gl);
   for (int i = threadIdx.x; i < A.n_gl; i += blockDim.x) {
-    const double nan = __builtin_nan("");
-    double2 xy = make_double2(nan, nan), zq = make_double2(nan, 0.0);
-    int ty = 0, k = i;
+    double2 xy = make_double2(0.0, 0.0), zq = xy;
+    int ty = -1, k = i;
     for (int c = 1; c < A.gv.n_comp; ++c) {
       const int ng = A.gv.seg[c].n_atoms, j = A.gv.seg[c].base + k;
       if (k >= 0 && k < ng && !(c == A.comp && A.g_molid[j] == A.new_molid)) {
@@ -1166,6 +1165,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 16 
     have = by_ins && whole ? ins : -1;
     // guest molecules (guest-guest)
     for (int j = lane; j < A.n_gl; j += 64) {
+      if (gty[j] < 0) continue;
       const double2 xy = gxy[j], zq = gzq[j];
       guest_pair<MIXED, CUBIC>(bc, ct, fr, coul, sq, xy.x - sx, xy.y - sy, zq.x - sz, zq.y, gty[j], v, r, o);
     }
