@@ -161,7 +161,7 @@ struct graspa_box {
   // scratch for per-move results
   double* d_part = nullptr;     // block partials
   size_t part_cap = 0;
-  double* h_part = nullptr;     // pinned mirror
+  double* h_part = nullptr;     // pinned mirror; per-move kernels write to it directly
   unsigned* d_ticket = nullptr;
 
   // Widom scratch
