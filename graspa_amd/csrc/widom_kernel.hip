@@ -752,7 +752,16 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 16 
   const int p_step = ranges ? 1 : nwave;
   int lo = 0;
   for (int pi = p_begin; pi < p_end; pi += p_step) {
-    lo = eval_sublist(pre, G, pi, lo, !ranges || pi == p_begin);
+    if (!ranges || pi == p_begin) {
+      // sub-list g holding point pi: the last g with pre[g] <= pi
+      int hi = G - 1;
+      lo = 0;
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if ((int)pre[mid] <= pi) lo = mid; else hi = mid - 1;
+      }
+    }
+    while (lo + 1 < G && (int)pre[lo + 1] <= pi) ++lo;
     const TrialPt P = list[(size_t)lo * chunk * per_ins + (pi - (int)pre[lo])];
     const double px = P.x, py = P.y, pz = P.z;
     const double sq = A.site_q[P.site];
@@ -893,9 +902,48 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 16 
         }
       }
     }
-    eval_guests<MIXED, CUBIC>(A, ct, fr, coul, sq, px, py, pz, lane, v, r, o);
-    n_eval += (unsigned long long)(n + A.n_guest);
-    eval_store<MIXED>(A, P.slot, P.ins, P.bit, coul, sq, lane, v, r, o, energy, mask);
+    // guest molecules (guest-guest), from memory (written out here, as is the
+    // sub-list search above: through the list kernel's functions this kernel
+    // spilled 20 more scalars around each point)
+    unsigned long long npair = (unsigned long long)n;
+    for (int c = 1; c < A.gv.n_comp; ++c) {
+      const int ng = A.gv.seg[c].n_atoms, base = A.gv.seg[c].base;
+      npair += (unsigned long long)ng;
+      for (int jj = lane; jj < ng; jj += 64) {
+        const int j = base + jj;
+        if (c == A.comp && A.g_molid[j] == A.new_molid) continue;
+        const int ta = A.g_type[j];
+        const double gq = A.g[3 * A.guest_cap + j];
+        double dx = A.g[j] - px, dy = A.g[A.guest_cap + j] - py, dz = A.g[2 * A.guest_cap + j] - pz;
+        if (MIXED)
+          pbc_rint<CUBIC>(dx, dy, dz, bc.cell, bc.inv);
+        else
+          pbc_fp64(dx, dy, dz, bc.cell, bc.inv, CUBIC ? 1 : 0);
+        const double rr = dx * dx + dy * dy + dz * dz;
+        if (rr < bc.cut_vdw2) {
+          const double4 ff = fr[ta];
+          const double e = MIXED ? lj_mixed_c(rr, ff.x, ff.y, ff.z) : lj_fp64(rr, ff.x, ff.y, ff.z);
+          o = o || (e > bc.overlap) || (rr < 0.01);
+          v += e;
+        }
+        if (coul && rr < bc.cut_coul2) {
+          if (MIXED) {
+            r = fma(gq, coul_table(ct, rr), r);    // scaled with the framework sum below
+          } else {
+            const double rd = sqrt(rr);
+            r += bc.prefactor * 1.0 * (gq * sq * erfc(bc.alpha * rd)) / rd;
+          }
+        }
+      }
+    }
+    n_eval += npair;
+    const double sv = wave_sum(v);
+    const double sr = coul ? (MIXED ? (bc.prefactor * sq) * wave_sum(r) : wave_sum(r)) : 0.0;
+    const bool ov = __any(o) != 0;
+    if (lane == 0) {
+      energy[P.slot] = make_double2(sv, sr);
+      if (ov) atomicOr(mask + P.ins, 1u << P.bit);
+    }
   }
   if (lane == 0 && n_eval) atomicAdd(&wg_eval, n_eval);
   __syncthreads();
@@ -1238,11 +1286,18 @@ __global__ __launch_bounds__(kInsWaves * 64) void widom_chain_kernel(const Widom
     b = (unsigned)__builtin_amdgcn_readfirstlane((int)b);
     if (on_lane) placed[b + __popcll(pm & lt)] = ins;
   };
-  // orientations of a live insertion whose first bead was placed (the whole
-  // wave; lane o * chain + a is orientation o's chain atom a)
-  auto orient = [&](const int ins, const uint64_t idx, const double fb0, const double fb1, const double fb2) {
-    const int o = lane / chain, a = lane - o * chain;
-    const bool act = lane < O * chain;
+  // orientations of live insertions whose first bead was placed, as many at a
+  // time as the wave has lanes for (three for ten orientations of two sites;
+  // 100,000 insertions into 750 atoms, 78,000 of them placed: one at a time
+  // 116 us, now 79):
+  // lane p * O * chain + o * chain + a is chain atom a of orientation o of the
+  // insertion in slot p, whose number and bead its lanes are given
+  const int oc = max(O * chain, 1), n_slot = 64 / oc;
+  const int p_slot = lane / oc, p_q = lane - p_slot * oc;
+  auto orient = [&](const bool on, const int ins, const double fb0, const double fb1, const double fb2) {
+    const int o = p_q / chain, a = p_q - o * chain;
+    const bool act = on && p_slot < n_slot;
+    const uint64_t idx = (uint64_t)(first_of(A) + ins);
     double p[3] = {0.0, 0.0, 0.0};
     bool hit = false;
     if (act) {
@@ -1257,11 +1312,14 @@ __global__ __launch_bounds__(kInsWaves * 64) void widom_chain_kernel(const Widom
     }
     const unsigned long long hits = __ballot(act && hit);
     const unsigned long long am = (1ull << chain) - 1ull;
-    uint32_t dead2 = 0u;
-    for (int oo = 0; oo < O; ++oo)
-      if ((hits >> (oo * chain)) & am) dead2 |= 1u << oo;
-    if (lane == 0) A.mask2[ins] = dead2;
-    const bool alive = act && !((dead2 >> o) & 1u);
+    const unsigned long long mine = hits >> (act ? p_slot * oc : 0);
+    const bool alive = act && !((mine >> (o * chain)) & am);
+    if (act && p_q == 0) {
+      uint32_t dead2 = 0u;
+      for (int oo = 0; oo < O; ++oo)
+        if ((mine >> (oo * chain)) & am) dead2 |= 1u << oo;
+      A.mask2[ins] = dead2;
+    }
     const unsigned long long al = __ballot(alive);
     if (al) {
       unsigned b = 0;
@@ -1323,11 +1381,18 @@ __global__ __launch_bounds__(kInsWaves * 64) void widom_chain_kernel(const Widom
       const unsigned long long okm = __ballot(fb_ok && rl == 0);
       to_finish(okm, fb_ok && rl == 0, ins);
       if (chain > 0) {
-        for (int r = 0; r < 4; ++r) {
-          if (!((okm >> (16 * r)) & 1ull)) continue;
-          const int ins_r = __builtin_amdgcn_readlane(ins, 16 * r);
-          orient(ins_r, (uint64_t)(first_of(A) + ins_r), readlane_d(S.fb[0], 16 * r), readlane_d(S.fb[1], 16 * r),
-                 readlane_d(S.fb[2], 16 * r));
+        // the placed rows (bits 0, 16, 32, 48), n_slot per pass in order
+        for (int done = 0, n_ok = __popcll(okm); done < n_ok; done += n_slot) {
+          int row_p = -1;
+          for (int r = 0, k = 0; r < 4; ++r)
+            if ((okm >> (16 * r)) & 1ull) {
+              if (k == done + p_slot) row_p = r;
+              ++k;
+            }
+          const int src = 16 * max(row_p, 0);
+          const int ins_p = __shfl(ins, src, 64);
+          const double f0 = __shfl(S.fb[0], src, 64), f1 = __shfl(S.fb[1], src, 64), f2 = __shfl(S.fb[2], src, 64);
+          orient(row_p >= 0, ins_p, f0, f1, f2);
         }
       }
     }
@@ -1366,7 +1431,7 @@ __global__ __launch_bounds__(kInsWaves * 64) void widom_chain_kernel(const Widom
         if (!fb_ok) failed_record(A, ins, 0);
       }
       to_finish(fb_ok ? 1ull : 0ull, fb_ok && lane == 0, ins);
-      if (fb_ok && chain > 0) orient(ins, idx, S.fb[0], S.fb[1], S.fb[2]);
+      if (fb_ok && chain > 0) orient(p_slot == 0, ins, S.fb[0], S.fb[1], S.fb[2]);
     }
   }
   if (st) atomicAdd(&wg_st, st);   // every lane's count (each lane screened its own trials)
