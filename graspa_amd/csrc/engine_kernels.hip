@@ -5,8 +5,8 @@
 //
 // Per-move work is small (tens of sites against ~10^3 atoms, ~10^3 k-vectors),
 // so these kernels are latency-shaped: one workgroup per probe site, sites and
-// force-field rows read through the scalar path, block partials returned to the
-// host in one copy.  The throughput path is the fused Widom kernel.
+// force-field rows read through the scalar path, block partials written to
+// pinned host memory (per-move calls) or returned in one copy (totals).  The throughput path is the fused Widom kernel.
 #include "device_math.hpp"
 #include "engine.hpp"
 #include "move_math.hpp"

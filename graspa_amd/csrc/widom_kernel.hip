@@ -11,13 +11,13 @@
 //      surviving trial sites to list 1;
 //   B  (one wave per trial site) full pair energies (LJ + real-space Coulomb,
 //      FP64 accumulation) of every site in the list, with the force-field rows,
-//      the real-space table and the framework staged in LDS; exact overlap
-//      flags;
-//   C  (one wave per live insertion)  first-bead selection; O orientations
+//      the real-space table and the framework staged in LDS, over all atoms or
+//      (FP64 form, wide cells) those of blocks in reach; exact overlap flags;
+//   C  (four live insertions per wave)  first-bead selection; O orientations
 //      of the template about the selected bead, one lane per orientation
 //      site, and their screen; survivors to list 2;
 //   D  = B on list 2;
-//   E  (one wave per live insertion)  orientation selection, Fourier-space energy
+//   E  (up to four placed insertions per wave)  orientation selection, Fourier-space energy
 //      of the selected molecule against the resident structure factors, W and
 //      the per-insertion record.
 // Two small kernels then sum the records in index order (deterministic sums).
@@ -1226,11 +1226,9 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 16 
   if (threadIdx.x == 0) stat_slot[blockIdx.x] = wg_eval;
 }
 
-// C: first-bead selection; orientations about the selected bead and their
-// overlap screen.  Workgroup g owns insertions [g*chunk, (g+1)*chunk).
-// C: one wave per live insertion (workgroup g takes the live sub-list of
-// first-bead workgroup g): first-bead selection from the evaluated trials,
-// the O orientations of the template about the selected bead (one lane per
+// C: workgroup g takes the live sub-list of first-bead workgroup g, up to four
+// insertions per wave: first-bead selection from the evaluated trials, the O
+// orientations of the template about the selected bead (one lane per
 // orientation site), their overlap screen, survivors appended to the
 // workgroup's sub-list of list 2.
 template <bool CUBIC>
