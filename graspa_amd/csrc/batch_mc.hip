@@ -2178,7 +2178,7 @@ int fill_slot(graspa_batch* bt, int i, const graspa_batch_box& in)
   h.ff64 = b->d_ff64;
   h.coul = b->d_coul; h.coul_n = b->coul_n;
   h.kstride = 1 + std::max(b->bc.kmax[0], std::max(b->bc.kmax[1], b->bc.kmax[2]));
-  h.kact = b->d_kact; h.ktemp_act = b->d_ktemp_act; h.n_active = b->bc.use_charges ? b->n_active : 0;
+  h.kact = b->d_kact; h.ktemp_act = b->d_ktemp_act; h.n_active = b->bc.use_charges ? b->n_kact : 0;
   hipFree(bt->skc[i]);
   bt->skc[i] = nullptr;
   if (h.n_active > 0) {

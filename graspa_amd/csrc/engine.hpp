@@ -141,6 +141,8 @@ struct graspa_box {
 
   // Ewald
   int nvec = 0, n_active = 0;
+  int n_kact = 0;               // entries of d_kact: those with a coefficient >= 0 (a left-handed cell, of
+                                // negative volume, has none)
   double* d_ktemp = nullptr;    // [nvec] prefactor * exp(-k^2/4a^2)/k^2 (x2 for kx>0), 0 if inactive
   double2* d_sk_fw = nullptr;
   double2* d_sk_ads = nullptr;

@@ -630,6 +630,7 @@ int graspa_box_create(const graspa_box_params* p, graspa_box** out)
       kact.push_back(make_int4(kx, ky, kz, k));
       tact.push_back(b->ktemp[k]);
     }
+    b->n_kact = (int)kact.size();
     const size_t na = std::max<size_t>(kact.size(), 1);
     rc = rc ? rc : hip_check(box_malloc(b, &b->d_kact, na * sizeof(int4)), "hipMalloc ewald");
     rc = rc ? rc : hip_check(box_malloc(b, &b->d_ktemp_act, na * sizeof(double)), "hipMalloc ewald");
@@ -1114,7 +1115,7 @@ int graspa_total_energy(graspa_box* b, graspa_energy* e)
   guest_view(b, &gv);
   // one partial per guest atom (pair sums) and per kBlock active k-vectors
   // (Fourier sums), read back in one copy
-  const size_t n_pair = 4 * (size_t)gv.total, n_four = 3 * (size_t)((b->n_active + kBlock - 1) / kBlock);
+  const size_t n_pair = 4 * (size_t)gv.total, n_four = 3 * (size_t)((b->n_kact + kBlock - 1) / kBlock);
   if (int rc = ensure_part(b, n_pair + n_four + 8)) return rc;
   int nb = 0, nk = 0;
   if (int rc = launch_total_pairs(b, b->d_part, &nb)) return rc;

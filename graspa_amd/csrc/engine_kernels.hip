@@ -442,10 +442,10 @@ __global__ __launch_bounds__(kBlock) void fourier_total_kernel(const int4* __res
 
 int launch_fourier_total(graspa_box* b, double* d_out, int* n_blocks)
 {
-  *n_blocks = (b->n_active + kBlock - 1) / kBlock;
+  *n_blocks = (b->n_kact + kBlock - 1) / kBlock;
   if (*n_blocks == 0) return GRASPA_OK;
   hipLaunchKernelGGL(fourier_total_kernel, dim3(*n_blocks), dim3(kBlock), 0, b->stream, b->d_kact, b->d_ktemp_act,
-                     b->n_active, b->d_sk_fw, b->d_sk_ads, d_out);
+                     b->n_kact, b->d_sk_fw, b->d_sk_ads, d_out);
   return hip_check(hipGetLastError(), "fourier_total launch");
 }
 

@@ -2288,7 +2288,7 @@ int launch_widom(graspa_box* b, int comp, int K, int O, double beta, int bias, d
   A.K = K; A.O = O; A.beta = beta; A.bias = bias; A.excl = excl; A.tail_de = tail_de;
   A.seed = seed; A.stream = stream; A.first_index = how.first_dev ? 0 : first_index; A.n_insert = n_insert;
   A.first_dev = how.first_dev;
-  A.n_kact = b->n_active;
+  A.n_kact = b->n_kact;
   A.kact = b->d_kact;
   A.ktemp_act = b->d_ktemp_act;
   A.sk_ads = b->d_sk_ads; A.sk_fw = b->d_sk_fw;
