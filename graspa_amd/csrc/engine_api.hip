@@ -243,6 +243,10 @@ static int build_blocks(graspa_box* b, const double w[3])
   const int n = b->n_fw, nb = (n + 15) / 16;
   const double rc = std::sqrt(bc.use_charges ? std::max(bc.cut_vdw2, bc.cut_coul2) : bc.cut_vdw2);
   const double wmin = std::min(std::fabs(w[0]), std::min(std::fabs(w[1]), std::fabs(w[2])));
+  // (images of a right-angled cell come from its diagonal alone: the lists,
+  // which wrap by the whole matrix, need the other entries to vanish)
+  const double off = std::fabs(bc.cell[1]) + std::fabs(bc.cell[2]) + std::fabs(bc.cell[5]);
+  if (bc.cubic && off > 1e-10) return GRASPA_OK;
   if (n == 0 || nb > 60000 || !(wmin * (1.0 + 1e-9) >= 2.0 * rc)) return GRASPA_OK;
   std::vector<std::array<double, 3>> pos(n);
   auto wrap = [&](const double* p, double* to) {

@@ -59,3 +59,33 @@ def test_block_lists_match_oracle(engine_mod, form, cell, n_fw, species, cut):
     assert np.all(err <= (1e-8 + 1e-10 * np.abs(ref["energy"][ok]) if form == "fp64" else 1e-3)), err.max()
     for other in shaped:
         assert np.array_equal(got["energy"], other["energy"]) and np.array_equal(got["rosen"], other["rosen"])
+
+
+def test_right_angled_form_with_entries_below_the_diagonal(engine_mod):
+    """Cells are taken as right-angled when the entries above the diagonal
+    (cell[3], cell[6], cell[7]) vanish, and images are then found from the
+    diagonal alone, whatever the entries below it: the pair kernel finds the
+    same images as the oracle in such a cell too (small atoms, so that no
+    overlap screen decides a trial)."""
+    from graspa_amd import synth
+    from oracle import binding as ob
+    s = synth.build(n_fw=300, L=30.0, species=("CO2",), seed=3, probs=dict(widom=1.0))
+    s.eps, s.sig = s.eps * 0.1, s.sig * 0.3
+    s.cell = np.array([30.0, 3.0, 0.0, 0.0, 30.0, 2.0, 0.0, 0.0, 30.0])
+    n = 60
+    o = ob.OracleSystem(s)
+    _, skf, ska, _, _, _ = o.ewald_total()
+    ref = ob.widom_records_to_numpy(o.widom_batch(1, ska, skf, seed=5, n_insert=n))
+    print("widom blocks, entries below the diagonal", flush=True)
+    box = engine_mod.Box(s, precision=engine_mod.GRASPA_FP64)
+    box.init_ewald()
+    intra, selfe = o.exclusion(1)
+    got = engine_mod.widom_results_to_numpy(box.widom_batch(1, n, seed=5, excl=intra + selfe)[0])
+    box.close()
+    assert ref["ok"].sum() > 20
+    assert np.array_equal(got["ok"], ref["ok"])
+    ok = ref["ok"] == 1
+    assert np.array_equal(got["first_bead"][ok], ref["first_bead"][ok])
+    assert np.array_equal(got["orientation"][ok], ref["orientation"][ok])
+    err = np.abs(got["energy"][ok] - ref["energy"][ok])
+    assert np.all(err <= 1e-8 + 1e-10 * np.abs(ref["energy"][ok])), err.max()
