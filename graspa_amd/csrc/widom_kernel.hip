@@ -1464,10 +1464,15 @@ __global__ __launch_bounds__(kInsWaves * 64) void widom_chain_kernel(const Widom
 // with 56 gathered bytes per k-vector and insertion the kernel was bound by
 // L2, 106 KB per insertion of a 40 x 40 x 27 A box (366 us of 20,000
 // insertions there, 406 us of 100,000 in a 24 A box, at a workgroup per CU 274
-// and 400; now 99 and 163).
-// M: sites per molecule (their row products are in registers).
+// and 400; 102 and 144 when this form came, 89 and 141 without spills).
+// M: sites per molecule (their row products are in registers).  Two waves per
+// SIMD at least (up to 256 VGPRs; M = 3 takes 202), so that nothing spills:
+// held to four (128 VGPRs, 284 B of scratch a lane) a batch of 1,000 took 28
+// us here instead of 12, a batch of 100,000 with 1,661 placed 23.5 instead of
+// 12.7; three (168 VGPRs, 120 B) took 14 and 16.7, and 73 and 130 us in the
+// two large batches above.
 template <int M>
-__global__ __launch_bounds__(kFinWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void widom_finish_kernel(const WidomArgs A)
+__global__ __launch_bounds__(kFinWaves * 64) __attribute__((amdgpu_waves_per_eu(2))) void widom_finish_kernel(const WidomArgs A)
 {
   extern __shared__ __align__(16) char dyn[];
   const BoxConst& bc = A.bc;
