@@ -80,6 +80,11 @@ void build_dead_map(const graspa_box* b, int site_type, std::vector<uint32_t>& b
     const double dz = cell[2] * g[0] + cell[5] * g[1] + cell[8] * g[2];
     vrad = std::max(vrad, 0.5 * std::sqrt(dx * dx + dy * dy + dz * dz));
   }
+  struct AxisVoxel {
+    int wrapped;
+    double near2, far2;
+  };
+  std::vector<AxisVoxel> axis[3];
   for (int i = 0; i < b->n_fw; ++i) {
     const double t2 = thr[b->fw_type[i]], tn2 = thr_near[b->fw_type[i]];
     if (!(t2 > 0.0)) continue;
@@ -93,23 +98,38 @@ void build_dead_map(const graspa_box* b, int site_type, std::vector<uint32_t>& b
       lo[a] = (int)std::floor((s[a] - ext) * nv[a]);
       hi[a] = (int)std::floor((s[a] + ext) * nv[a]);
     }
+    if (hi[0] < lo[0] || hi[1] < lo[1] || hi[2] < lo[2]) continue;
+    // per voxel index of an axis: the wrapped index and, in a right-angled
+    // cell, the squared distances along it to the voxel's nearest and farthest
+    // point (worked out here and not voxel by voxel: the divisions and
+    // remainders there took all of the time, 0.2 s for the two maps of a
+    // 1,536-atom cube of 24 A, 15% more or less with where the loop's code lay)
+    for (int a = 0; a < 3; ++a) {
+      axis[a].resize((size_t)(hi[a] - lo[a]) + 1);
+      for (int k = lo[a]; k <= hi[a]; ++k) {
+        AxisVoxel& v = axis[a][k - lo[a]];
+        v.wrapped = ((k % nv[a]) + nv[a]) % nv[a];
+        if (!ortho) continue;
+        const double lo_f = (double)k / nv[a], hi_f = (double)(k + 1) / nv[a];
+        const double d = s[a] < lo_f ? lo_f - s[a] : (s[a] > hi_f ? s[a] - hi_f : 0.0);
+        const double d0 = (lo_f - s[a]) * cell[4 * a], d1 = (hi_f - s[a]) * cell[4 * a];
+        v.near2 = d * d * cell[4 * a] * cell[4 * a];
+        v.far2 = std::max(d0 * d0, d1 * d1);
+      }
+    }
     for (int iz = lo[2]; iz <= hi[2]; ++iz)
-      for (int iy = lo[1]; iy <= hi[1]; ++iy)
+      for (int iy = lo[1]; iy <= hi[1]; ++iy) {
+        const AxisVoxel &vy = axis[1][iy - lo[1]], &vz = axis[2][iz - lo[2]];
+        const size_t row = (size_t)nv[0] * ((size_t)vy.wrapped + (size_t)nv[1] * vz.wrapped);
         for (int ix = lo[0]; ix <= hi[0]; ++ix) {
           const int ii[3] = {ix, iy, iz};
-          const int wx = ((ix % nv[0]) + nv[0]) % nv[0];
-          const int wy = ((iy % nv[1]) + nv[1]) % nv[1];
-          const int wz = ((iz % nv[2]) + nv[2]) % nv[2];
-          const size_t lin = (size_t)wx + (size_t)nv[0] * ((size_t)wy + (size_t)nv[1] * wz);
+          const AxisVoxel& vx = axis[0][ix - lo[0]];
+          const size_t lin = (size_t)vx.wrapped + row;
           if (free_bits) {
             // nearest point of the voxel to the atom
-            double near2 = 0.0;
+            double near2;
             if (ortho) {
-              for (int a = 0; a < 3; ++a) {
-                const double lo_f = (double)ii[a] / nv[a], hi_f = (double)(ii[a] + 1) / nv[a];
-                const double d = s[a] < lo_f ? lo_f - s[a] : (s[a] > hi_f ? s[a] - hi_f : 0.0);
-                near2 += d * d * cell[4 * a] * cell[4 * a];
-              }
+              near2 = vx.near2 + vy.near2 + vz.near2;
             } else {
               double df[3];
               for (int a = 0; a < 3; ++a) df[a] = ((double)ii[a] + 0.5) / nv[a] - s[a];
@@ -126,11 +146,7 @@ void build_dead_map(const graspa_box* b, int site_type, std::vector<uint32_t>& b
           double far2 = 0.0;
           if (ortho) {
             // axis-aligned voxel: the farthest corner takes the farther face on each axis
-            for (int a = 0; a < 3; ++a) {
-              const double d0 = ((double)ii[a] / nv[a] - s[a]) * cell[4 * a];
-              const double d1 = ((double)(ii[a] + 1) / nv[a] - s[a]) * cell[4 * a];
-              far2 += std::max(d0 * d0, d1 * d1);
-            }
+            far2 = vx.far2 + vy.far2 + vz.far2;
           } else {
             for (int corner = 0; corner < 8; ++corner) {
               double df[3];
@@ -145,6 +161,7 @@ void build_dead_map(const graspa_box* b, int site_type, std::vector<uint32_t>& b
           if (far2 >= t2) continue;
           bits[lin >> 5] |= 1u << (lin & 31);
         }
+      }
   }
 }
 

@@ -123,3 +123,59 @@ def test_free_voxels_hold_no_close_pair(name):
             rr = (dd * dd).sum(1)
             assert np.all(rr >= r2_ov[ty]), (p, rr.min())
         assert not _overlapping(s, cart[:200], site_type).any()
+
+
+def _overlap_r2(a4e, s2, shift, overlap, cut2):
+    """r^2 at which 4 eps (x^2 - x) - shift = overlap, x = (sigma / r)^6, at
+    least 0.01 and at most the cutoff: the engine's expression."""
+    thr = 0.01
+    if a4e > 0.0 and s2 > 0.0:
+        x = 0.5 * (1.0 + np.sqrt(1.0 + 4.0 * ((overlap + shift) / a4e)))
+        thr = max(thr, s2 / np.cbrt(x))
+    return min(thr, cut2)
+
+
+@pytest.mark.parametrize("edges", [(24.0, 24.0, 24.0), (13.0, 20.0, 9.5)])
+def test_maps_of_a_right_angled_cell_equal_their_definition_bit_for_bit(edges):
+    """Voxel by voxel in plain Python floats, the same operations in the same
+    order: farthest corner inside the overlap distance of some atom (marked),
+    nearest point beyond it for every atom (free).  Atoms at faces, corners
+    and outside the cell; one of no size."""
+    from graspa_amd import engine, synth
+    s = synth.config1(n_fw=7)
+    s.cell = np.array([edges[0], 0, 0, 0, edges[1], 0, 0, 0, edges[2]], dtype=float)
+    s.fw_pos = np.array([[0.0, 0.0, 0.0], [0.5, 0.31, 0.77], [0.9999, 0.2, 0.0], [1.37, -0.4, 2.2], [0.25, 0.25, 0.25],
+                         [0.7, 0.7, 0.7], [0.1, 0.9, 0.5]]) * np.array(edges)
+    s.setup_ewald()
+    T, site = s.ntypes, 4
+    dead, nv = engine.dead_map(s, site)
+    free, _ = engine.free_map(s, site)
+    want_dead = np.zeros(tuple(nv[::-1]), dtype=bool)
+    want_free = np.ones(tuple(nv[::-1]), dtype=bool)
+    eps, sig = np.asarray(s.eps).reshape(T, T), np.asarray(s.sig).reshape(T, T)
+    inv = [1.0 / e for e in edges]
+    for p, t in zip(s.fw_pos, s.fw_type):
+        r2 = _overlap_r2(4.0 * eps[t, site], sig[t, site] ** 2, np.asarray(s.shift).reshape(T, T)[t, site], s.overlap,
+                         s.cut_vdw ** 2)
+        f = [p[a] * inv[a] for a in range(3)]
+        ax = []
+        for a in range(3):
+            ext = np.sqrt(r2 * (1.0 + 1e-4)) / edges[a]
+            ks = range(int(np.floor((f[a] - ext) * nv[a])) - 1, int(np.floor((f[a] + ext) * nv[a])) + 2)
+            rows = []
+            for k in ks:
+                lo, hi = k / nv[a], (k + 1) / nv[a]
+                d = lo - f[a] if f[a] < lo else (f[a] - hi if f[a] > hi else 0.0)
+                rows.append((k % nv[a], d * d * edges[a] * edges[a], max(((lo - f[a]) * edges[a]) ** 2,
+                                                                         ((hi - f[a]) * edges[a]) ** 2)))
+            ax.append(rows)
+        for wz, nz, fz in ax[2]:
+            for wy, ny, fy in ax[1]:
+                for wx, nx, fx in ax[0]:
+                    if nx + ny + nz < r2 * (1.0 + 1e-4):
+                        want_free[wz, wy, wx] = False
+                    if fx + fy + fz < r2 * (1.0 - 1e-5):
+                        want_dead[wz, wy, wx] = True
+    assert want_dead.any() and not want_free.all()
+    assert np.array_equal(np.asarray(dead, dtype=bool), want_dead)
+    assert np.array_equal(np.asarray(free, dtype=bool), want_free)
