@@ -112,7 +112,7 @@ struct graspa_box {
   int cell_cap = 0;
   int use_cells = 0;
   // the framework in blocks of 16 neighbouring atoms for the pair kernel's
-  // block lists (WidomArgs), and whether it takes them
+  // block lists (WidomArgs), and whether it takes them; one allocation, at d_fwb
   double2* d_fwb = nullptr;
   int* d_fwb_type = nullptr;
   float4* d_blk = nullptr;
@@ -150,7 +150,8 @@ struct graspa_box {
   int4* d_kact = nullptr;       // active k-vectors: kx, ky, kz, index
   double* d_ktemp_act = nullptr;  // ktemp of the active k-vectors
   // the active k-vectors as rows (kx, ky) of k_z, -k_z pairs, 64 rows to a
-  // chunk (layout: WidomArgs), and the Widom finish kernel's coefficients
+  // chunk (layout: WidomArgs), and the Widom finish kernel's coefficients; one
+  // allocation, at d_ku
   int n_kchunk = 0, n_kpack = 0;
   int2* d_kchunk = nullptr;
   int* d_krow = nullptr;

@@ -236,7 +236,7 @@ void graspa::cell_widths(const graspa_box* b, double w[3])
 // 1330 us; 0.66: 559 against 531 a batch).
 static int build_blocks(graspa_box* b, const double w[3])
 {
-  box_free(b, b->d_fwb); box_free(b, b->d_fwb_type); box_free(b, b->d_blk);
+  box_free(b, b->d_fwb);
   b->d_fwb = nullptr; b->d_fwb_type = nullptr; b->d_blk = nullptr;
   b->n_blk = b->use_blocks = 0;
   const BoxConst& bc = b->bc;
@@ -248,7 +248,15 @@ static int build_blocks(graspa_box* b, const double w[3])
   const double off = std::fabs(bc.cell[1]) + std::fabs(bc.cell[2]) + std::fabs(bc.cell[5]);
   if (bc.cubic && off > 1e-10) return GRASPA_OK;
   if (n == 0 || nb > 60000 || !(wmin * (1.0 + 1e-9) >= 2.0 * rc)) return GRASPA_OK;
-  std::vector<std::array<double, 3>> pos(n);
+  // (a block is in reach of all points within the cutoff of one of its atoms,
+  // so the share is at least a sphere's)
+  const double most = bc.cubic ? 0.42 : 0.55, sphere = 4.0 / 3.0 * M_PI * rc * rc * rc;
+  if (b->precision == GRASPA_MIXED && sphere > most * std::fabs(b->volume)) return GRASPA_OK;
+  struct Atom {
+    double p[3];
+    int i;
+  };
+  std::vector<Atom> at(n);
   auto wrap = [&](const double* p, double* to) {
     for (int d = 0; d < 3; ++d) to[d] = p[d];
     for (int e = 0; e < 3; ++e) {
@@ -256,15 +264,16 @@ static int build_blocks(graspa_box* b, const double w[3])
       for (int d = 0; d < 3; ++d) to[d] += f * bc.cell[3 * e + d];
     }
   };
-  for (int i = 0; i < n; ++i) wrap(&b->fw_pos[3 * (size_t)i], pos[i].data());
-  std::vector<int> ord(n);
-  for (int i = 0; i < n; ++i) ord[i] = i;
+  for (int i = 0; i < n; ++i) {
+    wrap(&b->fw_pos[3 * (size_t)i], at[i].p);
+    at[i].i = i;
+  }
   auto bounds = [&](int from, int to, double lo[3], double hi[3]) {
-    for (int d = 0; d < 3; ++d) lo[d] = hi[d] = pos[ord[from]][d];
+    for (int d = 0; d < 3; ++d) lo[d] = hi[d] = at[from].p[d];
     for (int i = from + 1; i < to; ++i)
       for (int d = 0; d < 3; ++d) {
-        lo[d] = std::min(lo[d], pos[ord[i]][d]);
-        hi[d] = std::max(hi[d], pos[ord[i]][d]);
+        lo[d] = std::min(lo[d], at[i].p[d]);
+        hi[d] = std::max(hi[d], at[i].p[d]);
       }
   };
   std::vector<std::array<int, 2>> todo(1, {0, n});
@@ -279,17 +288,24 @@ static int build_blocks(graspa_box* b, const double w[3])
     for (int d = 1; d < 3; ++d)
       if (hi[d] - lo[d] > hi[ax] - lo[ax]) ax = d;
     const int mid = s[0] + 16 * (m / 2);
-    std::nth_element(ord.begin() + s[0], ord.begin() + mid, ord.begin() + s[1], [&](int x, int y) {
-      return pos[x][ax] < pos[y][ax] || (pos[x][ax] == pos[y][ax] && x < y);
+    std::nth_element(at.begin() + s[0], at.begin() + mid, at.begin() + s[1], [ax](const Atom& x, const Atom& y) {
+      return x.p[ax] < y.p[ax] || (x.p[ax] == y.p[ax] && x.i < y.i);
     });
     todo.push_back({s[0], mid});
     todo.push_back({mid, s[1]});
   }
-  const size_t np = 16 * ((size_t)nb + 1);
+  // one host and one device block: xy, zq (atoms), bounding boxes, types
+  const size_t np = 16 * ((size_t)nb + 1), bytes = np * (2 * sizeof(double2) + sizeof(int)) + 2 * (size_t)nb * sizeof(float4);
+  std::vector<char> host(bytes);
+  double2 *xy = reinterpret_cast<double2*>(host.data()), *zq = xy + np;
+  float4* blk = reinterpret_cast<float4*>(zq + np);
+  int* ty = reinterpret_cast<int*>(blk + 2 * (size_t)nb);
   const double nan = std::nan("");
-  std::vector<double2> xy(np, make_double2(nan, nan)), zq(np, make_double2(nan, 0.0));
-  std::vector<int> ty(np, 0);
-  std::vector<float4> blk(2 * (size_t)nb);
+  for (size_t i = 16 * (size_t)nb - 16; i < np; ++i) {
+    xy[i] = make_double2(nan, nan);
+    zq[i] = make_double2(nan, 0.0);
+    ty[i] = 0;
+  }
   double vol = 0.0, r_max = 0.0;
   const double margin = 2e-3 + 1e-6 * (std::fabs(bc.cell[0]) + std::fabs(bc.cell[4]) + std::fabs(bc.cell[8]));
   for (int k = 0; k < nb; ++k) {
@@ -302,30 +318,27 @@ static int build_blocks(graspa_box* b, const double w[3])
     }
     wrap(c, cw);
     for (int i = 0; i < m; ++i) {
-      const int a = ord[16 * k + i];
       const size_t to = 16 * (size_t)k + i;
-      xy[to] = make_double2(pos[a][0] + (cw[0] - c[0]), pos[a][1] + (cw[1] - c[1]));
-      zq[to] = make_double2(pos[a][2] + (cw[2] - c[2]), b->fw_q[a]);
-      ty[to] = b->fw_type[a];
+      const Atom& x = at[to];
+      xy[to] = make_double2(x.p[0] + (cw[0] - c[0]), x.p[1] + (cw[1] - c[1]));
+      zq[to] = make_double2(x.p[2] + (cw[2] - c[2]), b->fw_q[x.i]);
+      ty[to] = b->fw_type[x.i];
     }
     blk[2 * k] = make_float4((float)cw[0], (float)cw[1], (float)cw[2], 0.0f);
     blk[2 * k + 1] = make_float4((float)(h[0] + margin), (float)(h[1] + margin), (float)(h[2] + margin), 0.0f);
     r_max = std::max(r_max, std::sqrt(h[0] * h[0] + h[1] * h[1] + h[2] * h[2]) + 2.0 * margin);
     vol += 8.0 * (h[0] * h[1] * h[2] + (h[0] * h[1] + h[1] * h[2] + h[2] * h[0]) * rc) +
-           2.0 * M_PI * (h[0] + h[1] + h[2]) * rc * rc + 4.0 / 3.0 * M_PI * rc * rc * rc;
+           2.0 * M_PI * (h[0] + h[1] + h[2]) * rc * rc + sphere;
   }
   const float rcf = (float)(rc * (1.0 + 1e-6) + margin);
   // (beyond 0.99 widths a block could be in reach through a third image)
-  const double share = vol / nb / std::fabs(b->volume), most = bc.cubic ? 0.42 : 0.55;
+  const double share = vol / nb / std::fabs(b->volume);
   if ((b->precision == GRASPA_MIXED && share > most) || rcf + r_max > 0.99 * wmin) return GRASPA_OK;
-  int rcode = hip_check(box_malloc(b, &b->d_fwb, 2 * np * sizeof(double2)), "hipMalloc fw blocks");
-  rcode = rcode ? rcode : hip_check(box_malloc(b, &b->d_fwb_type, np * sizeof(int)), "hipMalloc fw blocks");
-  rcode = rcode ? rcode : hip_check(box_malloc(b, &b->d_blk, blk.size() * sizeof(float4)), "hipMalloc fw blocks");
-  rcode = rcode ? rcode : hip_check(hipMemcpy(b->d_fwb, xy.data(), np * sizeof(double2), hipMemcpyHostToDevice), "fw blocks upload");
-  rcode = rcode ? rcode : hip_check(hipMemcpy(b->d_fwb + np, zq.data(), np * sizeof(double2), hipMemcpyHostToDevice), "fw blocks upload");
-  rcode = rcode ? rcode : hip_check(hipMemcpy(b->d_fwb_type, ty.data(), np * sizeof(int), hipMemcpyHostToDevice), "fw blocks upload");
-  rcode = rcode ? rcode : hip_check(hipMemcpy(b->d_blk, blk.data(), blk.size() * sizeof(float4), hipMemcpyHostToDevice), "fw blocks upload");
-  if (rcode) return rcode;
+  if (hip_check(box_malloc(b, &b->d_fwb, bytes), "hipMalloc fw blocks") ||
+      hip_check(hipMemcpy(b->d_fwb, host.data(), bytes, hipMemcpyHostToDevice), "fw blocks upload"))
+    return GRASPA_ERR_HIP;
+  b->d_blk = reinterpret_cast<float4*>(b->d_fwb + 2 * np);
+  b->d_fwb_type = reinterpret_cast<int*>(b->d_blk + 2 * (size_t)nb);
   b->n_blk = nb;
   b->use_blocks = 1;
   b->blk_rcf = rcf;
@@ -438,15 +451,23 @@ int graspa::build_k_rows(graspa_box* b)
     }
   std::stable_sort(rows.begin(), rows.end(), [](const Row& x, const Row& y) { return x.top > y.top; });
   const int nch = ((int)rows.size() + 63) / 64;
-  std::vector<int2> chunk(std::max(nch, 1), make_int2(0, 0));
-  std::vector<int> row(64 * (size_t)std::max(nch, 1), 64 << 8);
   int n = 0;
-  for (int c = 0; c < nch; ++c) {
-    chunk[c] = make_int2(n, rows[64 * c].top);
-    n += 64 * (rows[64 * c].top + 1);
+  for (int c = 0; c < nch; ++c) n += 64 * (rows[64 * c].top + 1);
+  // one device block: the coefficients (written by the Widom kernels), then
+  // what is uploaded: ktemp and index pairs, chunks, rows
+  const size_t ne = (size_t)std::max(n, 1), nc = (size_t)std::max(nch, 1);
+  const size_t up = ne * (sizeof(double2) + sizeof(int2)) + nc * (sizeof(int2) + 64 * sizeof(int));
+  std::vector<char> host(up, 0);
+  double2* kt = reinterpret_cast<double2*>(host.data());
+  int2* idx = reinterpret_cast<int2*>(kt + ne);
+  int2* chunk = idx + ne;
+  int* row = reinterpret_cast<int*>(chunk + nc);
+  std::fill(idx, idx + ne, make_int2(-1, -1));
+  std::fill(row, row + 64 * nc, 64 << 8);
+  for (int c = 0, first = 0; c < nch; ++c) {
+    chunk[c] = make_int2(first, rows[64 * c].top);
+    first += 64 * (rows[64 * c].top + 1);
   }
-  std::vector<double2> kt((size_t)std::max(n, 1), make_double2(0.0, 0.0));
-  std::vector<int2> idx((size_t)std::max(n, 1), make_int2(-1, -1));
   for (size_t r = 0; r < rows.size(); ++r) {
     row[r] = rows[r].kx | ((rows[r].ky + 64) << 8);
     for (int kz = 0; kz <= rows[r].top; ++kz) {
@@ -462,17 +483,14 @@ int graspa::build_k_rows(graspa_box* b)
       }
     }
   }
+  if (hip_check(box_malloc(b, &b->d_ku, ne * sizeof(double4) + up), "hipMalloc k rows")) return GRASPA_ERR_HIP;
+  b->d_kt = reinterpret_cast<double2*>(b->d_ku + ne);
+  b->d_kidx = reinterpret_cast<int2*>(b->d_kt + ne);
+  b->d_kchunk = b->d_kidx + ne;
+  b->d_krow = reinterpret_cast<int*>(b->d_kchunk + nc);
   b->n_kchunk = nch;
   b->n_kpack = n;
-  int rc = hip_check(box_malloc(b, &b->d_kchunk, chunk.size() * sizeof(int2)), "hipMalloc k rows");
-  rc = rc ? rc : hip_check(box_malloc(b, &b->d_krow, row.size() * sizeof(int)), "hipMalloc k rows");
-  rc = rc ? rc : hip_check(box_malloc(b, &b->d_kt, kt.size() * sizeof(double2)), "hipMalloc k rows");
-  rc = rc ? rc : hip_check(box_malloc(b, &b->d_kidx, idx.size() * sizeof(int2)), "hipMalloc k rows");
-  rc = rc ? rc : hip_check(box_malloc(b, &b->d_ku, kt.size() * sizeof(double4)), "hipMalloc k rows");
-  rc = rc ? rc : hip_check(hipMemcpy(b->d_kchunk, chunk.data(), chunk.size() * sizeof(int2), hipMemcpyHostToDevice), "k rows upload");
-  rc = rc ? rc : hip_check(hipMemcpy(b->d_krow, row.data(), row.size() * sizeof(int), hipMemcpyHostToDevice), "k rows upload");
-  rc = rc ? rc : hip_check(hipMemcpy(b->d_kt, kt.data(), kt.size() * sizeof(double2), hipMemcpyHostToDevice), "k rows upload");
-  return rc ? rc : hip_check(hipMemcpy(b->d_kidx, idx.data(), idx.size() * sizeof(int2), hipMemcpyHostToDevice), "k rows upload");
+  return hip_check(hipMemcpy(b->d_kt, host.data(), up, hipMemcpyHostToDevice), "k rows upload");
 }
 
 #define GRASPA_CHECK_BOX(b) \
@@ -687,10 +705,10 @@ void graspa_box_destroy(graspa_box* b)
   box_free(b, b->d_ff64); box_free(b, b->d_ff32);
   box_free(b, b->d_fw); box_free(b, b->d_fw_type); box_free(b, b->d_fw_fix); box_free(b, b->d_fw_fixT);
   box_free(b, b->d_fws); box_free(b, b->d_fws_type); box_free(b, b->d_ctab);
-  box_free(b, b->d_fwb); box_free(b, b->d_fwb_type); box_free(b, b->d_blk);
+  box_free(b, b->d_fwb);
   box_free(b, b->d_g); box_free(b, b->d_g_type); box_free(b, b->d_g_molid); box_free(b, b->d_g_comp); box_free(b, b->d_g_fix);
   box_free(b, b->d_ktemp); box_free(b, b->d_sk_fw); box_free(b, b->d_sk_ads); box_free(b, b->d_sk_stage);
-  box_free(b, b->d_kchunk); box_free(b, b->d_krow); box_free(b, b->d_kt); box_free(b, b->d_kidx); box_free(b, b->d_ku);
+  box_free(b, b->d_ku);
   box_free(b, b->d_kact); box_free(b, b->d_ktemp_act); box_free(b, b->d_coul);
   free_dead_maps(b);
   for (Component& c : b->comps) box_free(b, c.d_chain);
