@@ -2055,10 +2055,12 @@ static int launch_eval(graspa_box* b, const WidomArgs& A, const TrialPt* list, c
     const int grid = eval_grid(b, kern, waves, lds, b->ev_per_cu);
     if (grid < 1) continue;
     *grid_out = grid;
-    if (timed) timing_begin(b, "widom");
+    // ("widom_list": of these launches, those that take block lists)
+    const char* family = b->use_blocks && b->timing.family == "widom_list" ? "widom_list" : "widom";
+    if (timed) timing_begin(b, family);
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(waves * 64), lds, b->stream, A, list, counts, groups, chunk,
                        per_ins, energy, mask, stat_slot);
-    if (timed) timing_end(b, "widom");
+    if (timed) timing_end(b, family);
     return hip_check(hipGetLastError(), "widom_eval_kernel launch");
   }
   return fail(GRASPA_ERR_UNSUPPORTED, "widom: no launch shape fits the LDS (pair energies)");

@@ -531,8 +531,9 @@ int  graspa_widom_autotune(graspa_box* box, int comp, int n_trial_pos, int n_tri
 /* ------------------------------------------------------------------------ */
 
 /* Kernel timing with HIP events on the box's stream.  While enabled, every
- * launch of the named kernel family ("widom", "site", "ewald") is bracketed by
- * events; graspa_timing_read returns the summed elapsed milliseconds and the
+ * launch of the named kernel family ("widom": the Widom pair-energy kernels,
+ * "widom_list": those of them that take block lists, "site", "ewald") is
+ * bracketed by events; graspa_timing_read returns the summed elapsed milliseconds and the
  * number of launches since graspa_timing_enable. */
 int  graspa_timing_enable(graspa_box* box, const char* family, int on);
 int  graspa_timing_read(graspa_box* box, double* total_ms, int64_t* launches);
