@@ -1,7 +1,8 @@
 """The pair queue of the batched driver's FP64 form against the oracle's
 trajectory: a skewed cell (no neighbour lists), separate LJ and Coulomb cutoffs
-either way round, uncharged molecules, and frameworks of less than one wave
-step, one atom more, and more than the workgroup's 512 lanes.  The same FP64
+either way round, uncharged molecules, frameworks of less than one wave step,
+one atom more, and more than the workgroup's 512 lanes, and frameworks that
+leave no room for the queue in LDS or that LDS does not hold.  The same FP64
 terms summed in another order: energy changes to 1e-10 of their size."""
 import numpy as np
 import pytest
@@ -14,6 +15,12 @@ pytestmark = pytest.mark.gpu
     (65, (24.0, 24.0, 24.0, 0, 0, 0), ("CO2",), (11.0, 12.0)),
     (513, (36.0, 30.0, 26.0, 0, 0, 0), ("N2",), (12.0, 10.0)),
     (300, (27.0, 27.0, 27.0, 0, 0, 0), ("methane",), (12.0, 12.0)),
+    # LDS holds the framework and the neighbour lists but no queue; the
+    # framework alone; or lists and queue, the framework read from memory
+    (3000, (56.0, 56.0, 56.0, 0, 0, 0), ("CO2",), (12.0, 12.0)),
+    (3500, (56.0, 56.0, 56.0, 0, 0, 0), ("CO2",), (12.0, 12.0)),
+    (3900, (56.0, 56.0, 56.0, 0, 0, 0), ("CO2",), (12.0, 12.0)),
+    (3000, (56.0, 56.0, 56.0, 3.0, -2.0, 1.5), ("CO2",), (12.0, 12.0)),
 ])
 def test_fp64_batch_matches_oracle(engine_mod, n_fw, cell, species, cut):
     from graspa_amd import synth
