@@ -42,7 +42,9 @@ def widom_flops(screened, evaluated, M, n_active_k, n_ok, charged=True):
     (trial site, atom) pair tested by the overlap screen (distance and test),
     52 per pair with full energies (33 uncharged), 16 per (k-vector, site) and
     12 per k-vector of the Fourier term of each completed insertion.  The pair
-    counts are the kernel's own work counters."""
+    counts are the kernel's own work counters; `evaluated` is sites times
+    atoms, all of them visited only by the all-atoms pair kernel, which every
+    box whose rate is reported here takes (fast form, 24 A cube)."""
     f = screened * SCREEN_FLOP + evaluated * (PAIR_FLOP if charged else PAIR_FLOP_UNCHARGED)
     if charged:
         f += n_ok * n_active_k * (16.0 * M + 12.0)

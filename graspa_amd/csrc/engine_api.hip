@@ -229,11 +229,14 @@ void graspa::cell_widths(const graspa_box* b, double w[3])
 // 2,100, 998 against 1621).  The fast form, whose pairs cost a third of the
 // FP64 form's, takes them where the blocks in reach of a site hold few of the
 // atoms (`share`, the mean volume of the points within the cutoff of a block
-// over the cell's): under 0.42 in cells with right angles (48 A cube,
-// 0.17: the two pair launches of 20,000 insertions 530 against 2510 us; 34 A
-// cube, 0.47, 622 against 579 us a batch; 24 A, 1, 677 against 454), under
-// 0.55 in others, whose plain form finds an image per pair (0.51: 710 against
-// 1330 us; 0.66: 559 against 531 a batch).
+// over the cell's): under 0.42 in cells with right angles (batches of 20,000
+// into empty cubes, lists against all atoms: 42 A, 0.25, 501 against 818 us;
+// 37 A, 0.37, 600 against 632; 35 A, 0.44, 542 against 525; 24 A, 1, 677
+// against 454), under 0.55 in others, whose plain form finds an image per pair
+// (0.54: 549 against 649 us; 0.65: 689 against 722; in another cell of 0.66
+// 559 against 531).  With guests, which the lists' kernel keeps in LDS, they
+// win further up (60 molecules: 33 A cube, 0.47, 1121 against 1420 us), but
+// the tables are made before a box's guests are known.
 static int build_blocks(graspa_box* b, const double w[3])
 {
   box_free(b, b->d_fwb);

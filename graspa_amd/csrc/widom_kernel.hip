@@ -176,7 +176,7 @@ struct WidomArgs {
   double* rec_w;              // [n_insert] W
   double* rec_e;              // [n_insert] dE
   int* rec_f;                 // [n_insert] bit 0 first bead placed, bit 1 complete
-  unsigned long long* stat;   // screened pairs, evaluated pairs (sums of stat_part)
+  unsigned long long* stat;   // screened pairs, sites evaluated times atoms (sums of stat_part)
   // LDS layout (bytes from the start of the dynamic area)
   int lds_thr, lds_tab;                 // screening kernels
   int lds_ffl, lds_coul, lds_fw, lds_list, lds_q, lds_g;   // pair-energy kernel (lds_coul is 0)
@@ -1222,6 +1222,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 16 
       guest_pair<MIXED, CUBIC>(bc, ct, fr, coul, sq, xy.x - sx, xy.y - sy, zq.x - sz, zq.y, gty[j], v, r, o);
     }
     if (A.n_gl == 0) eval_guests<MIXED, CUBIC>(A, ct, fr, coul, sq, sx, sy, sz, lane, v, r, o);
+    // (the pairs answered for, as in the all-atoms kernel, not the visits)
     n_eval += (unsigned long long)(A.n_fw + A.n_guest);
     eval_store<MIXED>(A, slot, ins, bit, coul, sq, lane, v, r, o, energy, mask);
   }
@@ -2100,14 +2101,15 @@ struct WidomBufs {
 
 // Screening grid of a batch: up to kMaxScreenGroups workgroups, each owning
 // a contiguous range of `chunk` insertions; the work lists and the live list
-// have a sub-list of chunk insertions per workgroup.  The first-bead, chain
-// and finish kernels hold one workgroup per CU, so a batch gets one for each
-// CU down to eight insertions a workgroup (at 384 insertions a workgroup,
-// 1,000 insertions ran on 3 CUs and 20,000 on 53: the three kernels took 31 /
-// 113 / 110 us of a batch of 1,000 and 42 / 145 / 365 us of a batch of 20,000
-// in a loaded box, now 11 / 18 / 18 and 18 / 38 / 274 us); a batch of more
-// than 384 a CU gets a multiple of the CU count: a few groups beyond it would
-// take a second round of the whole kernel.
+// have a sub-list of chunk insertions per workgroup.  The first-bead and chain
+// kernels hold one workgroup per CU, so a batch gets one for each CU down to
+// eight insertions a workgroup (at 384 insertions a workgroup, 1,000
+// insertions ran on 3 CUs and 20,000 on 53: the two kernels took 31 and 113 us
+// of a batch of 1,000 and 42 and 145 us of a batch of 20,000 in a loaded box,
+// 11 and 18, 18 and 38 us so; the finish kernel, up to kFinMaxPer workgroups a
+// list, went from 110 to 18 and from 365 to 274 us, and less since); a batch
+// of more than 384 a CU gets a multiple of the CU count: a few groups beyond
+// it would take a second round of the whole kernel.
 static void widom_grid(const graspa_box* b, int K, int n_insert, int* groups, int* chunk)
 {
   const long long per_group = 4LL * kFbWaves * (64 / K);

@@ -96,7 +96,9 @@ typedef struct {
   double n_first_bead;       /* insertions whose first bead was placed (orientations grown) */
   double n_ok;               /* insertions with a complete construction (W > 0)             */
   double screened_pairs;     /* work: (trial site, atom) pairs tested by the overlap screen */
-  double evaluated_pairs;    /* work: (trial site, atom) pairs with full energies           */
+  double evaluated_pairs;    /* work: trial sites with full energies times the atoms of the box
+                              * (framework and guests), also where the pair kernel's lists
+                              * leave most of them unvisited: pairs answered for, not visits */
 } graspa_widom_summary;
 
 /* ------------------------------------------------------------------------ */
@@ -465,11 +467,12 @@ int  graspa_widom_totals(graspa_box* box, graspa_widom_summary* totals, int rese
  * reference: it is for callers that cannot allocate device memory (code
  * under HIP graph capture, serving loops that forbid hipMalloc).  The
  * pipeline's scratch (trial masks, per-insertion state, work lists, energies,
- * records, partial sums) comes from one fixed 32 MiB block per device in the
- * library's static device memory instead of the box's buffers, and no
+ * records, partial sums) comes from one fixed block per device in the
+ * library's static device memory (40 MiB, of which a batch may count on 32)
+ * instead of the box's buffers, and no
  * certain-overlap voxel map is built (maps that earlier calls built are
  * used; without one the cell screen decides the same trials).  A batch that
- * needs more scratch than the block (about 18,000 CO2 insertions at 10 x 10
+ * needs more than 32 MiB of scratch (about 18,000 CO2 insertions at 10 x 10
  * trials on 256 CUs) is refused with GRASPA_ERR_ARG before any GPU work.
  * Results are those of graspa_widom_enqueue: the summary goes into the box's
  * running totals (graspa_widom_totals).  Every call on a device shares the
@@ -507,7 +510,8 @@ int  graspa_batch_block_stats(graspa_batch* batch, int i, graspa_block_stats* ou
 typedef struct {
   int waves;            /* waves per workgroup: 4, 8, 12 (default) or 16          */
   int per_cu;           /* workgroups per CU; 0 (default): as many as are resident */
-  int framework_lds;    /* 1 (default): framework staged in LDS when it fits; 0: read from L2 */
+  int framework_lds;    /* 1 (default): framework staged in LDS when it fits (with block lists and
+                         * per_cu 0: when it leaves room for two workgroups); 0: read from L2 */
 } graspa_eval_shape;
 
 /* Sets the box's launch shape (NULL: the default); GRASPA_ERR_ARG for a
