@@ -57,6 +57,7 @@ constexpr int kBGroup = 8;             // sites per pass over the atoms
 constexpr int kLocFw = 256;            // framework entries per wave
 constexpr int kLocG = 128;             // guest entries per wave
 constexpr int kPairQueue = 128;        // FP64 form: pairs that a wave queues at most (under 64, and a step's)
+constexpr int kQueueSites = 4;         // FP64 form: sites from which a pass queues its pairs
 constexpr int kBDrawTrial = 16;        // first trial draw
 constexpr int kBMaxDraws = kBDrawTrial + 9 * kBMaxTrial;   // K trials, O orientations, O retrace orientations
 
@@ -345,7 +346,13 @@ __device__ void block_sums(const BBox& B, const BState& S, const int bk, const i
 // sixth of the pairs of a 40 x 40 x 27 A box are inside, in nearly every wave
 // step of some site (10 cycles of that box, 2,304 atoms, 26 CO2 and more:
 // 30.3 and 25.3 ms).  Without room for the queues in LDS the pass runs as the
-// fast form's, whose pairs are a third as long.
+// fast form's, whose pairs are a third as long, and so does a pass over fewer
+// than kQueueSites sites: a wave then queues hardly more than it empties, and
+// where half of the atoms are inside the cutoff nothing is saved (an empty
+// 1,536-atom cube of 24 A, whose passes have one or two sites that the screen
+// left: 4.05 us a move without the queue, 4.17 with it in every pass, 4.09 so; from two
+// sites on it still lost 1%, from four nothing; a 28 A cube of 1,000 atoms with
+// molecules gains 1.19 times either way).
 template <bool CUBIC>
 __device__ uint32_t pair_queue(const BBox& B, const BState& S, BMove& L, const double* __restrict__ ffl,
                                const double* __restrict__ fwl, const double* __restrict__ gml, int* __restrict__ loc,
@@ -584,7 +591,7 @@ __device__ void pair_pass(const BBox& B, const BState& S, BMove& L, const double
   const int first = r * 64 + lane, stride = (w1 - w0) * 64;
   const int nf = B.n_fw, cap = B.guest_cap;
   uint32_t ovb = 0;
-  if (!MIXED && loc && L.queue) {
+  if (!MIXED && loc && L.queue && n_sites >= kQueueSites) {
     ovb = pair_queue<CUBIC>(B, S, L, ffl, fwl, gml, loc, use_loc, g0, cnt, r * 64, stride, ex_lo, ex_hi);
   } else
 #pragma unroll 1
